@@ -171,10 +171,10 @@ int syn_hip_attend_batch(syn_arena* arena, const syn_seq_desc* seqs, uint32_t n_
  * and head h, out_i,h = softmax_j(scale * q_i,h . k_j,h) v_j,h over j = 0..n-1.
  * Rows are grouped into `batch` independent images of n rows each (the
  * reference runs one image per run_rows call, S/models/clip.hpp:405-416).
- * f32 rows of images up to 16384 rows keep the reference's f32 arithmetic
- * (its fma chains, in its order); f16 rows, and longer f32 images, go to the
- * matrix cores as binary16 operands with binary16 probabilities. Softmax
- * and accumulation in f32, f32 output. */
+ * f32 rows of images up to 16384 rows keep f32 operands, products and sums
+ * throughout; f16 rows, and longer f32 images, go to the matrix cores as
+ * binary16 operands with binary16 probabilities. Softmax and accumulation
+ * in f32, f32 output. */
 typedef struct syn_self_desc {
     uint64_t q_offset;   /* batch*n rows of n_heads*head_dim, type in_dtype */
     uint64_t k_offset;

@@ -47,7 +47,7 @@ HIP_FLAGS = [
 # so their results go to VGPRs (no accumulator-register moves). The same for
 # the decode kernel measured no change.
 SOURCE_FLAGS = {"quant_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
-HIP_SOURCES = ["kv_append.hip", "decode.hip", "prefill.hip", "flash.hip", "generic.hip", "rope.hip", "ops.hip",
+HIP_SOURCES = ["kv_append.hip", "decode.hip", "prefill.hip", "flash.hip", "flash_f32.hip", "generic.hip", "rope.hip", "ops.hip",
                "quant.hip", "quant_gemm.hip", "capi.hip"]
 
 

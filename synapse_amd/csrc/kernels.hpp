@@ -258,12 +258,16 @@ hipError_t launch_bidirectional(const flash_args& a, uint32_t in_dtype, hipStrea
 hipError_t launch_generic_causal(const flash_args& a, uint32_t q_dtype, hipStream_t stream);
 hipError_t launch_generic_bidirectional(const flash_args& a, uint32_t in_dtype, hipStream_t stream);
 
-// Image-encoder attention on f32 rows in the reference's own f32 arithmetic
-// (no binary16 operands); images of up to self_f32_max_keys rows (the
-// probabilities of one query row sit in 64 KiB of LDS).
+// Image-encoder attention on f32 rows in f32 arithmetic (no binary16
+// operands); images of up to self_f32_max_keys rows (the probabilities of
+// one query row sit in 64 KiB of LDS).
 constexpr uint32_t self_f32_max_keys = 16384;
 bool self_f32_fits(uint32_t n);
 hipError_t launch_self_f32(const flash_args& a, hipStream_t stream);
+// The same on the f32 matrix cores (flash_f32.hip): head sizes in whole
+// 16-byte chunks, an image's rows below 2^31 bytes.
+bool self_f32_mfma_fits(const flash_args& a);
+hipError_t launch_self_f32_mfma(const flash_args& a, hipStream_t stream);
 
 // ---- RoPE -------------------------------------------------------------------
 struct rope_args {

@@ -1,0 +1,66 @@
+"""GPU parity of image-encoder attention on f32 rows: the f32 matrix-core
+kernel (flash_f32.hip) at the edges of its tiles, and the row-per-wave kernel
+(generic.hip) for head sizes that are not whole 16-byte chunks, against the
+oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import binding as orc
+from gpu_util import SYN_F32, Arena, self_attention
+from synapse_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+# Of the largest output: both sides sum in f32 (hd terms, then n), and each
+# f32 rounding of a random sum's partial is at most 6e-8 of it.
+BOUND = 2e-6
+
+
+@pytest.fixture(scope="module")
+def arena():
+    a = Arena(256 << 20)
+    yield a
+    a.close()
+
+
+# Keys go to the four waves in whole 16-row tiles, two per step: rows below,
+# at and above 1, 4 and 8 tiles, and a wave left without keys (n = 130 with 3
+# tiles a wave). Head sizes: one chunk, each group of the output's tiles (16,
+# 32, 64 dims) whole and cut, both ends of every compiled size, and 6 (the
+# row-per-wave kernel).
+@pytest.mark.parametrize("n,batch,heads,hd", [(1, 1, 1, 64), (15, 2, 3, 64), (16, 1, 1, 64), (17, 3, 1, 64),
+                                              (63, 1, 2, 64), (65, 2, 2, 64), (128, 1, 3, 64), (130, 1, 3, 64),
+                                              (257, 2, 9, 64), (729, 1, 2, 72), (40, 1, 2, 4), (40, 1, 2, 12),
+                                              (40, 2, 2, 32), (70, 1, 2, 36), (70, 1, 3, 80), (70, 1, 2, 84),
+                                              (70, 1, 2, 96), (70, 1, 2, 100), (70, 1, 2, 128), (70, 1, 2, 132),
+                                              (70, 1, 2, 192), (70, 1, 2, 196), (70, 1, 2, 256), (70, 1, 2, 6)])
+def test_image_f32(arena, n, batch, heads, hd):
+    g = wl.rng(1000 * hd + n)
+    q, k, v = (wl.normal(g, (batch * n, heads * hd)) for _ in range(3))
+    scale = float(np.float32(1) / np.sqrt(np.float32(hd)))
+    got = self_attention(arena, q, k, v, n, batch, heads, scale, SYN_F32)
+    for b in range(batch):
+        sl = slice(b * n, (b + 1) * n)
+        want = orc.self_attention(q[sl], k[sl], v[sl], heads, scale, threads=8)
+        assert np.abs(got[sl] - want).max() <= BOUND * np.abs(want).max(), b
+
+
+def test_image_f32_extreme_scores(arena):
+    """Scores far apart and rising along the keys (every step moves the max),
+    one key that outweighs the rest, and a row of NaN: as the oracle."""
+    n, heads, hd = 150, 2, 64
+    g = wl.rng(5)
+    q, k, v = (wl.normal(g, (n, heads * hd)) for _ in range(3))
+    k *= np.linspace(0.1, 30, n, dtype=np.float32)[:, None]
+    q[3] *= 100
+    q[7] = np.nan
+    got = self_attention(arena, q, k, v, n, 1, heads, 0.125, SYN_F32)
+    want = orc.self_attention(q, k, v, heads, 0.125, threads=8)
+    assert np.isnan(got[7]).all()
+    rows = np.arange(n) != 7
+    # A score of size s carries an error of s * 2^-24 * sqrt(hd) at most,
+    # which its exponential shows as a relative error.
+    top = np.abs((q[rows] @ k.T) * 0.125).max()
+    assert np.abs(got[rows] - want[rows]).max() <= max(BOUND, top * 2.0 ** -24 * 8) * np.abs(want[rows]).max()

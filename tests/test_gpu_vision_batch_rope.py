@@ -24,10 +24,9 @@ def arena():
 
 # ---- bidirectional ----------------------------------------------------------
 
-# f32 rows take a kernel with the reference's f32 arithmetic: the score and
-# output fma chains in the oracle's order; the exponential (device expf) and
-# the order of the double sum of the exponentials (per lane, then across
-# lanes) differ, which moves only the last bits.
+# f32 rows keep f32 operands, products and sums throughout; the order of the
+# sums and the exponential (device expf) differ from the oracle's, which moves
+# only the last bits.
 F32_BOUND = 2e-6
 
 
