@@ -43,11 +43,13 @@ HIP_FLAGS = [
     # Packed-FP32 instructions stay off on this pool (wrong results seen).
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-# Per-source additions: the int8 GEMM's products feed vector work directly,
-# so their results go to VGPRs (no accumulator-register moves). The same for
-# the decode kernel measured no change.
-SOURCE_FLAGS = {"quant_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Per-source additions: the int8 and f32 GEMMs' products feed vector work
+# directly, so their results go to VGPRs (no accumulator-register moves). The
+# same for the decode kernel measured no change.
+SOURCE_FLAGS = {"quant_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                "matmul_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 HIP_SOURCES = ["kv_append.hip", "decode.hip", "prefill.hip", "flash.hip", "flash_f32.hip", "generic.hip", "rope.hip", "ops.hip",
+               "matmul_f32.hip",
                "quant.hip", "quant_gemm.hip", "capi.hip"]
 
 

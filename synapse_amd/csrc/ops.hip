@@ -1,6 +1,5 @@
 // ops.hip — the rest of the reference's model graphs on the device: embedding
-// rows, RMSNorm and layer norm, F32 matrix products, the element-wise ops
-// between them (GELU included) and the pixel shuffle of the CLIP projector.
+// rows, RMSNorm and layer norm, the element-wise ops between them (GELU included) and the pixel shuffle of the CLIP projector.
 // With rope.hip and the attention kernels, a whole layer stack runs on the
 // GPU from one arena. These follow the reference's session executors
 // (S/graph/session.hpp:287-336, :375-378) and kernels
@@ -15,14 +14,6 @@
 namespace syn {
 
 namespace {
-
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        v += __shfl_xor(v, m, wave);
-    }
-    return v;
-}
 
 // out row i = table row tokens[i] (session::execute(op_embed), :331-336).
 __global__ __launch_bounds__(256) void embed_kernel(const float* table, float* out, embed_tokens t, uint32_t size) {
@@ -63,29 +54,6 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* in, const fl
     const float sc = scale_s;
     for (uint32_t e = threadIdx.x; e < size; e += 256) {
         y[e] = (x[e] * sc) * gamma[e];
-    }
-}
-
-// out[r][o] = sum_c w[o][c] x[r][c] (+ bias[o]): one wave per output element,
-// lanes striding over the columns (session::execute(op_matmul), :287-302;
-// op_add_bias, :306-312).
-__global__ __launch_bounds__(256) void matmul_kernel(const float* w, const float* x, const float* bias, float* out,
-                                                     uint32_t rows, uint32_t cols) {
-    const uint32_t o = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const uint32_t r = blockIdx.y;
-    if (o >= rows) {
-        return;  // wave-uniform
-    }
-    const uint32_t ln = threadIdx.x & 63;
-    const float* wr = w + static_cast<std::size_t>(o) * cols;
-    const float* xr = x + static_cast<std::size_t>(r) * cols;
-    float acc = 0.0f;
-    for (uint32_t c = ln; c < cols; c += 64) {
-        acc += wr[c] * xr[c];
-    }
-    acc = wave_sum_f(acc);
-    if (ln == 0) {
-        out[static_cast<std::size_t>(r) * rows + o] = bias != nullptr ? acc + bias[o] : acc;
     }
 }
 
@@ -294,13 +262,6 @@ hipError_t launch_softmax(const float* in, float* out, uint32_t n, uint32_t size
 hipError_t launch_rms_norm(const float* in, const float* gamma, float* out, uint32_t n, uint32_t size, float eps,
                            hipStream_t stream) {
     rms_norm_kernel<<<n, 256, 0, stream>>>(in, gamma, out, size, eps);
-    return hipGetLastError();
-}
-
-hipError_t launch_matmul(const float* w, const float* x, const float* bias, float* out, uint32_t n, uint32_t rows,
-                         uint32_t cols, hipStream_t stream) {
-    const dim3 grid((rows + 3) / 4, n);
-    matmul_kernel<<<grid, 256, 0, stream>>>(w, x, bias, out, rows, cols);
     return hipGetLastError();
 }
 
