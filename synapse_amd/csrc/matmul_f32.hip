@@ -35,6 +35,8 @@ __device__ __forceinline__ float mf_wave_sum(float v) {
 // and this one is held to the reference's logits to 1e-4 by the golden
 // models; 16-byte loads would take another. What the loads need instead is
 // number: 16 weight loads (4 KB) in flight per wave and eight waves per SIMD.
+// One row of 16000 x 2048 21.5 us (6.1 TB/s), 5632 x 2048 8.8, 2048 x 5632
+// 8.9 us; with one load in flight per lane 39.4, 17.7 and 41.0.
 // Row resources end at the row, so columns past it add zeros.
 template <int NR>
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* w, const float* x, const float* bias, float* out,
@@ -102,7 +104,11 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* w, const flo
 // zero in four chains of 8 columns, which are added to one of four running
 // sums: short chains instead of one of cols, so that the rounding error stays
 // that of one wave per output (gemv_f32_kernel): against 64 bits at 768
-// columns @@ and 7.1e-8 of the result's norm.
+// columns 7.0e-8 and 7.1e-8 of the result's norm. (One chain of 32 a stage
+// and one running sum: 1.0e-7, and 42.1 us where this takes 45.7.)
+//
+// Bound by the f32 matrix rate: 1024 rows of 3072 x 768 45.7 us a call (106
+// TFLOP/s of 157; 1317 us with one wave per output), 4096 rows 109 TFLOP/s.
 template <int WM, int WN, int WK>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* w, const float* x, const float* bias, float* out,
                                                        uint32_t n, uint32_t rows, uint32_t cols, uint32_t row_tiles) {
@@ -236,9 +242,9 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* w, const flo
 // The matrix-core kernel's time for few rows is its stages' latency (6 ns per
 // column), the other's grows with n rows cols (0.15 us per million): they
 // meet at n rows = 40000. us per call, one wave per weight row against
-// tiles: 768 x 3072 weights 12.5 / 19.9 at 32 rows, 22.7 / 20.2 at 64; 3072 x
-// 768 5.9 / 6.7 at 8 and 9.7 / 7.0 at 16; 1152 x 588 7.3 / 7.1 at 32. Fewer
-// than 8 rows would leave three quarters of a tile empty.
+// tiles: 768 x 3072 weights 12.3 / 19.9 at 32 rows, 22.7 / 22.8 at 64; 3072 x
+// 768 5.9 / 6.7 at 8 and 9.7 / 8.0 at 16; 1152 x 588 7.3 / 7.7 at 32, 12.7 /
+// 8.1 at 64. Fewer than 8 rows would leave three quarters of a tile empty.
 bool on_matrix_cores(uint32_t n, uint32_t rows, uint32_t cols) {
     // (The tiled kernel copies whole 16-byte chunks of a row.)
     return n >= 8 && uint64_t{n} * rows >= 40000 && cols % 4 == 0;
@@ -256,10 +262,10 @@ hipError_t launch_matmul(const float* w, const float* x, const float* bias, floa
         };
         // The largest tile whose count still fills the 256 CUs (the waves
         // then split the columns). us per call for 64 x 64, 32 x 64 and
-        // 32 x 32 tiles: 1024 rows of 3072 x 768 45.4, 50.4, 60.4 (768 tiles
-        // of 64 x 64); 512 rows 31.8, 28.3, 33.7 (384 and 768); 729 rows of
-        // 768 x 3072 61.1, 57.9, 53.1 (144, 276, 552); 257 rows of 768 x 768
-        // 18.0, 11.6, 8.1.
+        // 32 x 32 tiles (with one running sum): 1024 rows of 3072 x 768 45.4,
+        // 50.4, 60.4 (768 tiles of 64 x 64); 512 rows 31.8, 28.3, 33.7 (384
+        // and 768); 729 rows of 768 x 3072 61.1, 57.9, 53.1 (144, 276, 552);
+        // 257 rows of 768 x 768 18.0, 11.6, 8.1.
         if (tiles(64, 64) >= 512) {
             go(gemm_f32_kernel<2, 2, 1>, 64, 64);
         } else if (tiles(32, 64) >= 384) {

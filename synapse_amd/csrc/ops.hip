@@ -1,5 +1,6 @@
 // ops.hip — the rest of the reference's model graphs on the device: embedding
-// rows, RMSNorm and layer norm, the element-wise ops between them (GELU included) and the pixel shuffle of the CLIP projector.
+// rows, RMSNorm and layer norm, the element-wise ops between them (GELU
+// included) and the pixel shuffle of the CLIP projector.
 // With rope.hip and the attention kernels, a whole layer stack runs on the
 // GPU from one arena. These follow the reference's session executors
 // (S/graph/session.hpp:287-336, :375-378) and kernels
