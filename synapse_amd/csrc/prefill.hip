@@ -858,11 +858,396 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
     }
 }
 
+// ---- short runs over a long cache: keys split inside the block -----------------------
+//
+// A prompt's chunk gives the pair kernel few blocks (509 queries of 32 heads:
+// 64 on 256 CUs), each with all the cached keys to walk. Here a block of 8
+// waves takes 64 queries of one head, four wave groups of two waves a quarter
+// of the key tiles each, a wave 32 queries: four times the blocks, and each
+// walks a quarter of the keys. A group has its own two LDS stages of 32-key
+// tiles (a whole tile of 64 keys in two stages for four groups would not
+// fit); the four partial (max, sum, O) meet in LDS at the end, in a fixed
+// order. One barrier per tile: tile j has landed and tile j - 1 is read, so
+// tile j + 1's copy goes out ahead of tile j's products.
+//
+// 509 queries after 7683 rows (32 heads on 8, hd 128): 112 us, 590 TFLOP/s
+// (263 us as pairs). Copies alone take 81 us (each tile serves 64 queries, so
+// the CUs read 1.07 GB through L2) and the products and softmax alone 83:
+// with one block per CU in step they overlap only in part.
+constexpr int ps_bq = 64;  // queries per block
+constexpr int ps_bk = 32;  // keys per LDS tile
+constexpr int ps_groups = 4;
+
+template <int HD, bool QF16>
+__global__ __launch_bounds__(512, 2) void prefill_split_kernel(const flash_args a) {
+    constexpr int NS = HD / 16;
+    constexpr int NT = HD / 32;
+    constexpr int HSPAN = HD / 2;
+    constexpr int KCPR = HD / 8;
+    constexpr int KROWC = KCPR + 1;
+    constexpr int VROWC = ps_bk / 8 + 1;
+    constexpr int TK = (ps_bk * KROWC + 63) / 64;
+    constexpr int TV = (HD * VROWC + 63) / 64;
+    constexpr int TT = TK + TV;
+    constexpr int STAGE = TT * 1024;
+    // The merge takes NT * 16 + 2 floats per lane of all 8 waves.
+    static_assert(2 * ps_groups * STAGE >= 8 * (NT * 16 + 2) * 256, "merge does not fit the stage buffers");
+    __shared__ __attribute__((aligned(16))) char lds[2 * ps_groups * STAGE];
+
+    const int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = w >> 1;  // key group
+    const int wq = w & 1;    // 32-query half of the block
+    const int ln = tid & 63;
+    const int H = ln >> 5;
+    const int qi = ln & 31;
+    const uint32_t hd = a.hd;
+    // Heads fastest (an XCD keeps whole KV heads, as in the pair kernel), the
+    // latest queries, with the most keys, first.
+    const uint32_t n_qt = (a.n + ps_bq - 1) / ps_bq;
+    const uint32_t qt = n_qt - 1 - blockIdx.x / a.n_heads;
+    const uint32_t h = pf_head(blockIdx.x % a.n_heads, a.n_heads);
+    const uint32_t g = h / a.group;
+    const float c = a.scale_log2e;
+
+    const uint32_t q_first = qt * ps_bq;
+    const uint32_t q_row0 = q_first + 32 * wq;
+    const uint32_t my_q = q_row0 + qi;
+    const uint32_t my_pos = a.pos + my_q;
+    const uint32_t kv_end = a.pos + min(a.n, q_first + ps_bq);         // keys this block needs
+    const uint32_t wave_last_pos = a.pos + min(a.n - 1, q_row0 + 31);  // causal horizon of the wave
+    const uint32_t n_tiles = (kv_end + ps_bk - 1) / ps_bk;
+    // A block with queries before position 64 takes its first two tiles as
+    // one in group 0: those queries take their softmax whole (probabilities).
+    const bool whole_block = a.pos + q_first < pf_bk;
+    const uint32_t per = max((n_tiles + ps_groups - 1) / ps_groups, whole_block ? 2u : 1u);
+    const uint32_t tile0 = grp * per;
+    const uint32_t cnt = tile0 < n_tiles ? min(per, n_tiles - tile0) : 0;
+
+    h8 qv[NS];
+#pragma unroll
+    for (int st = 0; st < NS; ++st) {
+        const uint32_t d0 = H * HSPAN + 8 * st;
+        qv[st] = my_q < a.n && d0 < hd ? pf_load_q<QF16>(a.q, static_cast<std::size_t>(my_q) * a.q_row + h * hd + d0)
+                                       : as_h8(zero_u4());
+    }
+
+    // Tile copies as in the kernels above, over the group's two waves; vc[i]
+    // is the key chunk of a V^T copy (8 keys), or 8 for none.
+    constexpr int CPW = (TT + 1) / 2;
+    uint32_t coff[CPW], vc[CPW];
+#pragma unroll
+    for (int i = 0; i < CPW; ++i) {
+        const uint32_t j = wq + 2 * i;
+        coff[i] = buffer_oob;
+        vc[i] = 8;
+        if (j < TK) {
+            const uint32_t L = 64 * j + ln;
+            const uint32_t r = L / KROWC, cc = L % KROWC;
+            if (r < ps_bk && cc < KCPR && 8 * cc < hd) {
+                coff[i] = r * a.row * 2 + cc * 16;
+            }
+        } else if (j < TT) {
+            const uint32_t L = 64 * (j - TK) + ln;
+            const uint32_t d = L / VROWC, cc = L % VROWC;
+            if (cc < ps_bk / 8 && d < hd) {
+                coff[i] = d * a.ctx_stride * 2 + cc * 16;
+                vc[i] = cc;
+            }
+        }
+    }
+    const _Float16* k_head = a.k + g * hd;
+    const _Float16* v_head = a.vt + static_cast<std::size_t>(g) * hd * a.ctx_stride;
+    const uint32_t k_bytes = kv_end * a.row * 2 - g * hd * 2;
+    const uint32_t v_bytes = hd * a.ctx_stride * 2;
+    char* const stages = lds + grp * 2 * STAGE;
+    const auto stage = [&](uint32_t j) __attribute__((always_inline)) { return stages + (j & 1) * STAGE; };
+    // Tile tile0 + j into its stage (a tile at or past kv_end lands as zeros).
+    const auto issue = [&](uint32_t j) __attribute__((always_inline)) {
+        const uint32_t t0 = (tile0 + j) * ps_bk;
+        const rsrc k_res = make_rsrc(k_head + static_cast<std::size_t>(t0) * a.row,
+                                     t0 < kv_end ? k_bytes - t0 * a.row * 2 : 0u);
+        const rsrc v_res = make_rsrc(v_head + t0, t0 < kv_end ? v_bytes - t0 * 2 : 0u);
+        const bool last = t0 + ps_bk > kv_end;
+        const uint32_t base = pf_copy_base(stage(j), wq);
+#pragma unroll
+        for (int i = 0; i < CPW; ++i) {
+            const uint32_t jj = wq + 2 * i;
+            if (jj < TK) {
+                pf_copy(k_res, base + 2048 * i, coff[i]);
+            } else if (jj < TT) {
+                pf_copy(v_res, base + 2048 * i, last && vc[i] < 8 && t0 + 8 * vc[i] >= kv_end ? buffer_oob : coff[i]);
+            }
+        }
+    };
+    // After tile j landed: the V^T chunk straddling kv_end holds stale halves
+    // past it (zero probability times a stale non-finite half would be NaN);
+    // the lane that copied it zeroes them.
+    const auto tail = [&](uint32_t j) __attribute__((always_inline)) {
+        const uint32_t t0 = (tile0 + j) * ps_bk;
+        if (t0 + ps_bk <= kv_end || t0 >= kv_end || kv_end % 8 == 0) {
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < CPW; ++i) {
+            const uint32_t jj = wq + 2 * i;
+            if (jj >= TK && jj < TT && vc[i] == (kv_end - t0) / 8) {
+                _Float16* chunk = reinterpret_cast<_Float16*>(stage(j) + 1024 * jj + 16 * ln);
+                for (uint32_t k = kv_end % 8; k < 8; ++k) {
+                    chunk[k] = 0;
+                }
+            }
+        }
+    };
+
+    f16v o[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            o[n][i] = 0.0f;
+        }
+    }
+    // This lane's query: running max (lazy, as above), and this lane half's
+    // share of the sum.
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    const auto scores = [&](uint32_t t0, const char* sk, f16v& sc) __attribute__((always_inline)) {
+        const char* krow = sk + (pf_slice_key(qi) * KROWC + H * (KCPR / 2)) * 16;
+        h8 kop[NS];
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            kop[st] = *reinterpret_cast<const h8*>(krow + 16 * st);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            sc[i] = 0.0f;
+        }
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            sc = mfma32(kop[st], qv[st], sc);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, NS, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, NS, 0);
+        if (t0 + ps_bk - 1 > a.pos + q_row0 || t0 + ps_bk > kv_end) {
+            // (as the pair kernel masks: register i holds key 16 (i / 8) + 8 H + i % 8)
+            const int lim = static_cast<int>(max(min(my_pos + 1, kv_end), t0) - t0) - 8 * H;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                sc[i] = 16 * (i >> 3) + (i & 7) < lim ? sc[i] : -INFINITY;
+            }
+        }
+    };
+    const auto raise = [&](float tmax) __attribute__((always_inline)) {
+        const bool grow = (tmax - m_run) * c > 8.0f;
+        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+            const float m_new = grow ? tmax : m_run;
+            const float alpha = grow ? fast_exp2((m_run - m_new) * c) : 1.0f;
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    o[n][i] *= alpha;
+                }
+            }
+        }
+        return (m_run == -INFINITY ? 0.0f : m_run) * c;
+    };
+    const auto output = [&](const char* sv, const h8& p0, const h8& p1) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const char* vrow = sv + ((32 * n + qi) * VROWC + H) * 16;
+            o[n] = mfma32(*reinterpret_cast<const h8*>(vrow), p0, o[n]);
+            o[n] = mfma32(*reinterpret_cast<const h8*>(vrow + 32), p1, o[n]);
+        }
+    };
+    const auto compute = [&](uint32_t j) __attribute__((always_inline)) {
+        const uint32_t t0 = (tile0 + j) * ps_bk;
+        if (q_row0 >= a.n || t0 > wave_last_pos) {
+            return;
+        }
+        const char* sk = stage(j);
+        f16v sc;
+        scores(t0, sk, sc);
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            tmax = fmaxf(tmax, sc[i]);
+        }
+        const float mc = raise(max32(tmax));
+        h8 pv[2];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            pv[i >> 3][i & 7] = to_h(fast_exp2(sc[i] * c - mc));
+        }
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) {
+                l_run = add_pair(h2{pv[s2][i], pv[s2][i + 1]}, l_run);
+            }
+        }
+        output(sk + 1024 * TK, pv[0], pv[1]);
+    };
+    // Group 0's first two tiles of a whole_block, as one of 64 keys.
+    const auto compute_first = [&]() __attribute__((always_inline)) {
+        if (q_row0 >= a.n) {
+            return;
+        }
+        f16v sc[2];
+        scores(0, stage(0), sc[0]);
+        scores(ps_bk, stage(1), sc[1]);
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                tmax = fmaxf(tmax, sc[e][i]);
+            }
+        }
+        const float mc = raise(max32(tmax));
+        h8 pv[4];
+        const bool whole = probabilities(0, a.pos + q_row0, my_pos, mc, sc, pv, c);
+        float psum = 0.0f;
+#pragma unroll
+        for (int s2 = 0; s2 < 4; ++s2) {
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) {
+                psum = add_pair(h2{pv[s2][i], pv[s2][i + 1]}, psum);
+            }
+        }
+        l_run = whole ? 0.5f : l_run + psum;  // (two lane halves: 1 together)
+        output(stage(0) + 1024 * TK, pv[0], pv[1]);
+        output(stage(1) + 1024 * TK, pv[2], pv[3]);
+    };
+
+    // Every group runs `per` steps, one barrier each, whatever its count.
+    const auto landed = [&](uint32_t j) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(pf_vmcnt(0));
+        if (j < cnt) {
+            tail(j);
+        }
+        pf_barrier();
+    };
+    issue(0);
+    uint32_t j = 0;
+    if (whole_block) {  // block-uniform
+        issue(1);
+        landed(0);
+        if (grp == 0) {
+            tail(1);
+            pf_barrier();
+            compute_first();
+        } else {
+            pf_barrier();
+            if (cnt > 0) {
+                compute(0);
+            }
+            if (cnt > 1) {
+                tail(1);
+            }
+        }
+        pf_barrier();
+        if (grp != 0 && cnt > 1) {
+            compute(1);
+        }
+        pf_barrier();
+        j = 2;
+        if (j < per) {
+            issue(j);
+        }
+    }
+    for (; j < per; ++j) {
+        landed(j);
+        if (j + 1 < cnt) {
+            issue(j + 1);
+        }
+        if (j < cnt) {
+            compute(j);
+        }
+    }
+
+    // ---- merge the groups' partials ------------------------------------------------
+    // Float f of lane (w, ln) at float f * 512 + 64 w + ln: o[n][i] is f = 16 n + i,
+    // then the max and the sum. Group grp then merges output tiles grp,
+    // grp + 4, ... of its queries.
+    l_run = sum32(l_run);
+    __builtin_amdgcn_s_waitcnt(pf_vmcnt(0));
+    pf_barrier();
+    float* part = reinterpret_cast<float*>(lds) + 64 * wq + ln;
+    {
+        float* mine = part + 128 * grp;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                mine[(16 * n + i) * 512] = o[n][i];
+            }
+        }
+        mine[16 * NT * 512] = m_run;
+        mine[(16 * NT + 1) * 512] = l_run;
+    }
+    pf_barrier();
+    if (my_q >= a.n) {
+        return;
+    }
+    float m = -INFINITY, f[ps_groups], l = 0.0f;
+#pragma unroll
+    for (int v = 0; v < ps_groups; ++v) {
+        f[v] = part[128 * v + 16 * NT * 512];
+        m = fmaxf(m, f[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < ps_groups; ++v) {
+        f[v] = f[v] == -INFINITY ? 0.0f : fast_exp2((f[v] - m) * c);
+        l += part[128 * v + (16 * NT + 1) * 512] * f[v];
+    }
+    const float inv = 1.0f / l;
+    float* out = a.out + static_cast<std::size_t>(my_q) * a.q_row + h * hd;
+    for (uint32_t n = grp; n < NT; n += ps_groups) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const uint32_t d = 32 * n + 8 * b + 4 * H;
+            if (d < hd) {
+                f4 r{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                    for (int v = 0; v < ps_groups; ++v) {
+                        r[i] += part[128 * v + (16 * n + 4 * b + i) * 512] * f[v];
+                    }
+                    r[i] *= inv;
+                }
+                *reinterpret_cast<f4*>(out + d) = r;
+            }
+        }
+    }
+}
+
 template <int HD>
 hipError_t launch_hd(const flash_args& a, uint32_t dtype, hipStream_t stream) {
     if constexpr (HD <= 128) {
         // Two wave groups' stages fit LDS up to hd 128.
         const dim3 grid(a.n_heads * ((a.n + 2 * pf_bq - 1) / (2 * pf_bq)));
+        // Where those blocks leave CUs idle, blocks of 64 queries with the
+        // keys split four ways, up to two of them per CU. us per call, pairs
+        // against split keys (32 heads on 8, hd 128): 509 queries after 7683
+        // rows 263 / 112, after 1000 53 / 25, after none 22.3 / 13.4; 64 after
+        // 7683 127 / 91; 1024 after 7683 (512 blocks) 275 / 211, 1100 after
+        // 7683 (576) 269 / 283. Below 128 keys there is little to split: 64
+        // queries after none 6.9 / 8.2, after 100 9.6 / 9.4.
+        const uint32_t cus = device_cu_count();
+        const dim3 fine(a.n_heads * ((a.n + ps_bq - 1) / ps_bq));
+        if (grid.x < cus && fine.x <= 2 * cus && a.kv_len >= 128) {
+            if (dtype == 1) {
+                prefill_split_kernel<HD, true><<<fine, 512, 0, stream>>>(a);
+            } else {
+                prefill_split_kernel<HD, false><<<fine, 512, 0, stream>>>(a);
+            }
+            return hipGetLastError();
+        }
         if (dtype == 1) {
             prefill_pair_kernel<HD, true><<<grid, 512, 0, stream>>>(a);
         } else {

@@ -158,3 +158,37 @@ def test_prefill_is_causal(arena):
                               cfg.scale))
     assert np.array_equal(outs[0][:100], outs[1][:100])
     assert not np.array_equal(outs[0][100:], outs[1][100:])
+
+
+# The split-key kernel (few blocks as pairs, at least 128 keys): both sides of
+# that rule, queries before position 64 (whole softmax over two tiles) with
+# one to four key tiles, tile counts that leave groups short or empty, ends on
+# and off 8- and 32-key edges, a second half of a block without queries, head
+# counts that are no multiple of 8, every compiled head size whole and cut.
+@pytest.mark.parametrize("n_heads,n_kv,hd,n,pos", [
+    (4, 2, 128, 2, 125), (4, 2, 128, 2, 126), (4, 2, 128, 128, 0), (4, 2, 128, 127, 1), (8, 8, 32, 200, 0),
+    (14, 2, 64, 33, 95), (14, 2, 64, 64, 64), (14, 2, 64, 65, 160), (3, 1, 96, 32, 255), (3, 1, 96, 70, 63),
+    (6, 3, 40, 65, 103), (5, 5, 72, 97, 160), (28, 4, 128, 31, 700), (32, 8, 128, 509, 131), (7, 1, 24, 130, 40),
+])
+@pytest.mark.parametrize("dtype", [SYN_F32, SYN_F16])
+def test_prefill_split_keys(arena, n_heads, n_kv, hd, n, pos, dtype):
+    got, want, (dk, dv), ok_k, ok_v = _prefill(arena, n_heads, n_kv, hd, n, pos, seed=n + hd + pos, dtype=dtype)
+    assert np.array_equal(dk, ok_k[:pos + n]) and np.array_equal(dv, ok_v[:pos + n])
+    assert_close(got, want, what=f"split keys {n_heads}/{n_kv}/{hd} n={n} pos={pos}")
+
+
+def test_prefill_split_keys_ignores_rows_past_the_run(arena):
+    """Cache rows at and past pos + n that hold NaN leave the output as is."""
+    n_heads, n_kv, hd, n, pos = 4, 2, 128, 61, 90
+    row = n_kv * hd
+    g = wl.rng(91)
+    kc, vc = (wl.to_f16_bits(wl.normal(g, (256, row))) for _ in range(2))
+    q = wl.normal(g, (n, n_heads * hd))
+    outs = []
+    for bits in (0, 0x7E00):
+        kc[pos + n:] = vc[pos + n:] = bits
+        c = capi.kv_state(arena, 256, n_kv, hd)
+        capi.upload_cache(arena, c, kc, vc)
+        outs.append(attention(arena, c, scratch_for(arena, n_heads, n_kv, hd, 256), q, None, None, pos, n_heads,
+                              hd ** -0.5, append=False))
+    assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
