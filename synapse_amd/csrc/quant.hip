@@ -232,7 +232,9 @@ __global__ __launch_bounds__(512) void gemv_q_kernel(const uint8_t* w, const flo
             // into a dword: the resource starts at the dword.
             const uint8_t* rp = w + static_cast<std::size_t>(o0 + t / nb * o_step) * wrow;
             x.delta = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(rp) & 3);
-            x.r = make_rsrc(rp - x.delta, wrow + x.delta);
+            // It ends on a dword too: the range check is per dword, and a row
+            // of an odd number of blocks may end inside one.
+            x.r = make_rsrc(rp - x.delta, (wrow + x.delta + 3) & ~3u);
             x.k = t % nb;
         }
         return x;

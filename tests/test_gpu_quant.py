@@ -184,3 +184,19 @@ def test_matmul_q_rejects_bad_shapes(arena):
     assert lib().syn_hip_matmul_q(arena.handle, ctypes.byref(d)) != 0
     assert lib().syn_hip_matmul_q_act_bytes(Q4_K, 2, 512) == 2 * 2 * 292
     assert lib().syn_hip_matmul_q_act_bytes(Q8_0, 1, 100) == 0
+
+
+@pytest.mark.parametrize("t", [Q4_0, Q5_0, Q8_0, Q6_K])
+@pytest.mark.parametrize("n", [1, 2, 5])
+def test_matmul_q_odd_block_counts(arena, t, n):
+    """Rows of an odd number of blocks (800 or 768 columns) end inside a dword
+    when they start on one: their last two bytes are read too. Every output
+    within 1e-5 of sum |w| |x^|, as above."""
+    rows, cols = 7, 768 if t == Q6_K else 800
+    rng = np.random.default_rng(50 + t)
+    raw = random_blocks(t, rows, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    out, act = matmul_q(arena, raw, t, x, rows, cols)
+    w = qh.dequantize(raw, t).reshape(rows, cols).astype(np.float64)
+    xa = np.stack([qh.dequantize_act(a, qh.act_type(t)) for a in act.reshape(n, -1)]).astype(np.float64)
+    assert np.all(np.abs(out - xa @ w.T) <= 1e-5 * np.maximum(np.abs(xa) @ np.abs(w).T, 1.0))
