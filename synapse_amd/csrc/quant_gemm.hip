@@ -149,10 +149,12 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(const uint8_t* w, const uin
     const uint32_t wave_rows = o0 < rows ? min(32u, rows - o0) : 0;
     const uint8_t* wp = w + static_cast<std::size_t>(min(o0, rows - 1)) * wrow;
     const uint32_t delta = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wp) & 3);
-    const rsrc wr = make_rsrc(wp - delta, wave_rows * wrow + delta);
+    // (to a whole dword: the range check is per dword, and the last row may
+    // end inside one)
+    const rsrc wr = make_rsrc(wp - delta, (wave_rows * wrow + delta + 3) & ~3u);
     const uint32_t wlane = li * wrow + delta;  // this lane's row inside the resource
     // The block's 64 activation rows; rows past n read zeros.
-    const rsrc ar = make_rsrc(act + static_cast<std::size_t>(t0) * arow, min(gq_n, n - t0) * arow);
+    const rsrc ar = make_rsrc(act + static_cast<std::size_t>(t0) * arow, (min(gq_n, n - t0) * arow + 3) & ~3u);
 
     float acc[2][16];
 #pragma unroll

@@ -187,7 +187,7 @@ def test_matmul_q_rejects_bad_shapes(arena):
 
 
 @pytest.mark.parametrize("t", [Q4_0, Q5_0, Q8_0, Q6_K])
-@pytest.mark.parametrize("n", [1, 2, 5])
+@pytest.mark.parametrize("n", [1, 2, 5, 33])
 def test_matmul_q_odd_block_counts(arena, t, n):
     """Rows of an odd number of blocks (800 or 768 columns) end inside a dword
     when they start on one: their last two bytes are read too. Every output
