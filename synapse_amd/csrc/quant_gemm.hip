@@ -14,7 +14,9 @@
 //   Q6_K               per 256-block: (d yd) (float(sum_k sc_k sumi_k) - 32 sum_k sc_k bsum_k)
 //
 // so each block's integers are ggml's and results differ from its gemv only
-// by float association. Three kernels:
+// by float association. The kernels, chosen in launch_gemm_q:
+// - gemm_r16_kernel (all formats, up to 32 activation rows) and gemm_ks_kernel
+//   (all formats, few 32 x 32 tiles): the columns split over a block's waves.
 // - gemm_q4k_kernel (Q4_K): a workgroup (4 waves) owns 128 weight rows x 64
 //   activation rows; a wave 32 weight rows (one per lane, the product's B
 //   operand) against the 64 activation rows (two A operands). Each
@@ -752,6 +754,55 @@ __device__ __forceinline__ void lds_chunk_words(const uint8_t* p, uint32_t (&d)[
     }
 }
 
+// Block b of a stage: this lane's weight row window at WR against G tiles of
+// 32 activation rows (windows at A, scales da[b][row]).
+template <uint32_t T, int b, int G>
+__device__ __forceinline__ void k32_block(const uint8_t* WR, const uint8_t* A, const float* da, uint32_t H, uint32_t li,
+                                          float (&acc)[G][16]) {
+                // d_w at byte BB b of the row, then the block's quants.
+                const float dw = half_bits(*reinterpret_cast<const uint16_t*>(WR + block_bytes<T> * b));
+                uint32_t q[4];
+                if constexpr (T == qtype_q8_0) {  // this lane half's 16 bytes at 34 b + 2 + 16 H
+                    constexpr uint32_t C = (34 * b + 2) / 16 * 16, M = (34 * b + 2) % 16;
+                    lds_chunk_words<M>(WR + C + 16 * H, q);
+                } else if constexpr (T == qtype_q4_0) {  // 16 bytes at 18 b + 2, this lane half's nibbles
+                    constexpr uint32_t C = (18 * b + 2) / 16 * 16, M = (18 * b + 2) % 16;
+                    uint32_t qs[4];
+                    lds_chunk_words<M>(WR + C, qs);
+    #pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        q[j] = sext4((qs[j] >> (4 * H)) & 0x0F0F0F0Fu);
+                    }
+                } else {  // Q5_0: the 32 high bits at 22 b + 2, then 16 bytes
+                    constexpr uint32_t C = (22 * b + 2) / 16 * 16, M = (22 * b + 2) % 16;
+                    uint32_t hq[5];
+                    lds_chunk_words<M>(WR + C, hq);
+    #pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        q[j] = sext5(((hq[1 + j] >> (4 * H)) & 0x0F0F0F0Fu) | spread4((hq[0] >> (16 * H + 4 * j)) & 0xF));
+                    }
+                }
+                const i4v qv = {static_cast<int>(q[0]), static_cast<int>(q[1]), static_cast<int>(q[2]),
+                                static_cast<int>(q[3])};
+    #pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    constexpr uint32_t CA = (34 * b + 2) / 16 * 16, MA = (34 * b + 2) % 16;
+                    uint32_t av[4];
+                    lds_chunk_words<MA>(A + (32 * g + li) * k32_awin + CA + 16 * H, av);
+                    const i4v a = {static_cast<int>(av[0]), static_cast<int>(av[1]), static_cast<int>(av[2]),
+                                   static_cast<int>(av[3])};
+                    const i16v cm = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, qv, i16v{}, 0, 0, 0);
+    #pragma unroll
+                    for (int qd = 0; qd < 4; ++qd) {
+                        const f4 d4 = *reinterpret_cast<const f4*>(da + 32 * G * b + 32 * g + 8 * qd + 4 * H);
+    #pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            acc[g][4 * qd + k] += static_cast<float>(cm[4 * qd + k]) * (dw * d4[k]);
+                        }
+                    }
+                }
+}
+
 template <uint32_t T>
 __global__ __launch_bounds__(256, 4) void gemm_qb32_kernel(const uint8_t* w, const uint8_t* act, const float* bias,
                                                            float* out, uint32_t n, uint32_t rows, uint32_t cols) {
@@ -839,52 +890,8 @@ __global__ __launch_bounds__(256, 4) void gemm_qb32_kernel(const uint8_t* w, con
         const uint8_t* S = lds[U & 1];
         const uint8_t* WR = S + (32 * wv + li) * WWIN;
         const float* da = reinterpret_cast<const float*>(S + KD);
-        const auto block = [&]<int b>() __attribute__((always_inline)) {
-            // d_w at byte BB b of the row, then the block's quants.
-            const float dw = half_bits(*reinterpret_cast<const uint16_t*>(WR + BB * b));
-            uint32_t q[4];
-            if constexpr (T == qtype_q8_0) {  // this lane half's 16 bytes at 34 b + 2 + 16 H
-                constexpr uint32_t C = (34 * b + 2) / 16 * 16, M = (34 * b + 2) % 16;
-                lds_chunk_words<M>(WR + C + 16 * H, q);
-            } else if constexpr (T == qtype_q4_0) {  // 16 bytes at 18 b + 2, this lane half's nibbles
-                constexpr uint32_t C = (18 * b + 2) / 16 * 16, M = (18 * b + 2) % 16;
-                uint32_t qs[4];
-                lds_chunk_words<M>(WR + C, qs);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    q[j] = sext4((qs[j] >> (4 * H)) & 0x0F0F0F0Fu);
-                }
-            } else {  // Q5_0: the 32 high bits at 22 b + 2, then 16 bytes
-                constexpr uint32_t C = (22 * b + 2) / 16 * 16, M = (22 * b + 2) % 16;
-                uint32_t hq[5];
-                lds_chunk_words<M>(WR + C, hq);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    q[j] = sext5(((hq[1 + j] >> (4 * H)) & 0x0F0F0F0Fu) | spread4((hq[0] >> (16 * H + 4 * j)) & 0xF));
-                }
-            }
-            const i4v qv = {static_cast<int>(q[0]), static_cast<int>(q[1]), static_cast<int>(q[2]),
-                            static_cast<int>(q[3])};
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                constexpr uint32_t CA = (34 * b + 2) / 16 * 16, MA = (34 * b + 2) % 16;
-                uint32_t av[4];
-                lds_chunk_words<MA>(S + KA + (32 * g + li) * k32_awin + CA + 16 * H, av);
-                const i4v a = {static_cast<int>(av[0]), static_cast<int>(av[1]), static_cast<int>(av[2]),
-                               static_cast<int>(av[3])};
-                const i16v cm = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, qv, i16v{}, 0, 0, 0);
-#pragma unroll
-                for (int qd = 0; qd < 4; ++qd) {
-                    const f4 d4 = *reinterpret_cast<const f4*>(da + 64 * b + 32 * g + 8 * qd + 4 * H);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        acc[g][4 * qd + k] += static_cast<float>(cm[4 * qd + k]) * (dw * d4[k]);
-                    }
-                }
-            }
-        };
-        block.template operator()<0>();
-        block.template operator()<1>();
+        k32_block<T, 0, 2>(WR, S + KA, da, H, li, acc);
+        k32_block<T, 1, 2>(WR, S + KA, da, H, li, acc);
     }
 
     const uint32_t o = o0 + li;
@@ -902,7 +909,775 @@ __global__ __launch_bounds__(256, 4) void gemm_qb32_kernel(const uint8_t* w, con
         }
     }
 }
+
+// ---- few activation rows: columns split over the block's waves --------------------------
+//
+// With 32 activation rows the kernels above fill a handful of CUs (a 4096-row
+// product is 32 or 64 blocks), each walking every column, and the GEMV decodes
+// every weight once per four rows. Here a block owns 32 weight rows x 32
+// activation rows and its four waves every fourth unit of the columns (a
+// 256-block of Q4_K / Q6_K, two 32-blocks of the others), so a product has
+// rows / 32 blocks per 32 activation rows whatever its column count, and each
+// walks a quarter of it. A wave stages its own units through its own LDS (the
+// same whole-line copies and layouts as above, ks_stages deep) and waits for
+// nothing but its copies: no barrier until the four partial sums meet, in a
+// fixed order. The block sums are the same exact integers. 64 rows against
+// Q4_K 4096 x 14336: 23 us a call (93 in the 128 x 64 tiles), Q6_K 34 (121),
+// Q8_0 41 (239).
+// gemm_q4k_kernel's block for one tile of 32 activation rows: this lane's
+// weight row (its 144 bytes at Wl) against the rows of the stage at S, qs at A
+// (256 bytes a row, 16-byte chunk k of a row at k ^ (row % 16)), the 16 sums
+// of 16 at BS (32 bytes a row), the scales at D. (A function of its own: with
+// the large tile calling it too, that kernel was scheduled 1 to 2 % slower.)
+template <uint32_t A, uint32_t BS, uint32_t D>
+__device__ __forceinline__ void k4_block(const uint8_t* S, const uint8_t* Wl, uint32_t H, uint32_t li,
+                                         float (&acc)[16]) {
+    // d, dmin and the 8 (scale, min) pairs of this lane's weight row, as
+    // bytes: sc 0..3, sc 4..7, m 0..3, m 4..7 (ggml's get_scale_min_k4).
+    const u4 hdr = *reinterpret_cast<const u4*>(Wl);
+    const float wd = half_bits(hdr[0] & 0xFFFF), wdmin = half_bits(hdr[0] >> 16);
+    const uint32_t sc[2] = {hdr[1] & 0x3F3F3F3Fu, (hdr[3] & 0x0F0F0F0Fu) | ((hdr[1] >> 2) & 0x30303030u)};
+    const uint32_t mn[2] = {hdr[2] & 0x3F3F3F3Fu, ((hdr[3] >> 4) & 0x0F0F0F0Fu) | ((hdr[2] >> 2) & 0x30303030u)};
+
+    i16v a1, a2;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {  // sub-blocks 2t (low nibbles) and 2t + 1 (high)
+        const u4 qw = *reinterpret_cast<const u4*>(Wl + 16 + 32 * t + 16 * H);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t s = 2 * t + e;
+            const uint32_t sl = byte_pair(sc[s / 4] & 0x07070707u, s % 4);
+            const uint32_t sh = byte_pair((sc[s / 4] >> 3) & 0x07070707u, s % 4);
+            i4v p1, p2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t nib = (qw[j] >> (4 * e)) & 0x0F0F0F0Fu;
+                p1[j] = static_cast<int>(mul_u16x2(nib, sl));
+                p2[j] = static_cast<int>(mul_u16x2(nib, sh));
+            }
+            const u4 av = *reinterpret_cast<const u4*>(S + A + li * 256 + 16 * ((2 * s + H) ^ (li & 15)));
+            const i4v a = {static_cast<int>(av[0]), static_cast<int>(av[1]), static_cast<int>(av[2]),
+                           static_cast<int>(av[3])};
+            a1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, p1, s == 0 ? i16v{} : a1, 0, 0, 0);
+            a2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, p2, s == 0 ? i16v{} : a2, 0, 0, 0);
+        }
+    }
+
+    // mins: B = m of sub-blocks 4H .. 4H + 3, each for its two sums of 16.
+    const uint32_t mh = mn[H];
+    h8 mb;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const _Float16 m = static_cast<_Float16>(static_cast<float>((mh >> (8 * j)) & 0xFF));
+        mb[2 * j] = m;
+        mb[2 * j + 1] = m;
+    }
+    const u4 bv = *reinterpret_cast<const u4*>(S + BS + 32 * li + 16 * H);
+    h8 ab;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        ab[2 * j] = static_cast<_Float16>(static_cast<int16_t>(bv[j] & 0xFFFF));
+        ab[2 * j + 1] = static_cast<_Float16>(static_cast<int16_t>(bv[j] >> 16));
+    }
+    const f16v fm = mfma32(ab, mb, f16v{});
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t r0 = 8 * q + 4 * H;
+        const f4 yd = *reinterpret_cast<const f4*>(S + D + 4 * r0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = 4 * q + k;
+            const int isum = a1[i] + (a2[i] << 3);
+            acc[i] += yd[k] * (wd * static_cast<float>(isum) - wdmin * fm[i]);
+        }
+    }
+}
+
+// gemm_q6k_kernel's block likewise: this lane's weight row from byte o of its
+// window at RB.
+template <uint32_t A, uint32_t BS, uint32_t D>
+__device__ __forceinline__ void k6_block(const uint8_t* S, const uint8_t* RB, uint32_t o, uint32_t H, uint32_t li,
+                                         float (&acc)[16]) {
+    // 16 signed scales and d.
+    const u4 s4 = *reinterpret_cast<const u4*>(RB + 192);
+    const uint32_t s5 = *reinterpret_cast<const uint32_t*>(RB + 208);
+    const uint32_t s6 = *reinterpret_cast<const uint32_t*>(RB + 212);
+    const uint32_t sc[4] = {__builtin_amdgcn_alignbyte(s4[1], s4[0], o), __builtin_amdgcn_alignbyte(s4[2], s4[1], o),
+                            __builtin_amdgcn_alignbyte(s4[3], s4[2], o), __builtin_amdgcn_alignbyte(s5, s4[3], o)};
+    const float wd = half_bits(__builtin_amdgcn_alignbyte(s6, s5, o) & 0xFFFF);
+
+    // Four groups (hf, kq) of four products (kh, e) each: a group's
+    // products are issued before the previous group's results are scaled,
+    // so the matrix cores run under the integer multiply-adds.
+    int isum[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        isum[i] = 0;
+    }
+    i16v cm[2][4];
+    int sck[2][4];
+    const auto scale_group = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                // |sums| < 2^17 and |sc| <= 128: 24-bit multiplies are
+                // exact. The empty asm keeps one multiply-add per product
+                // (else the adds are regrouped into separate multiplies
+                // and three-input adds).
+                int v = __mul24(sck[t & 1][j], cm[t & 1][j][i]) + isum[i];
+                asm volatile("" : "+v"(v));
+                isum[i] = v;
+            }
+        }
+    };
+    uint64_t qh[2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int hf = t / 2, kq = t % 2;
+        if (kq == 0) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                qh[e] = lds_bytes8(RB + 128 + 32 * hf + 16 * e + 8 * H, o);
+            }
+        }
+        uint64_t ql[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            ql[e] = lds_bytes8(RB + 64 * hf + 32 * kq + 16 * e + 8 * H, o);
+        }
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh) {
+            const int k4 = 2 * kh + kq, s = 4 * hf + k4;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const uint64_t lo = (ql[e] >> (4 * kh)) & 0x0F0F0F0F0F0F0F0Full;
+                const uint64_t hi = k4 < 3 ? (qh[e] << (4 - 2 * k4)) & 0x3030303030303030ull
+                                           : (qh[e] >> 2) & 0x3030303030303030ull;
+                const long bw = static_cast<long>(lo | hi);
+                const long a = *reinterpret_cast<const long*>(S + A + li * 256 +
+                                                              16 * ((2 * s + e) ^ (li & 15)) + 8 * H);
+                cm[t & 1][2 * kh + e] = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, bw, i16v{}, 0, 0, 0);
+                const uint32_t k = 2 * s + e;  // sub-block of 16
+                sck[t & 1][2 * kh + e] = static_cast<int8_t>((sc[k / 4] >> (8 * (k % 4))) & 0xFF);
+            }
+        }
+        if (t > 0) {
+            scale_group(t - 1);
+        }
+    }
+    scale_group(3);
+
+    // The offset term: A = the activation sums of 16, B = sc, both for
+    // k = 8H .. 8H + 7.
+    const u4 bv = *reinterpret_cast<const u4*>(S + BS + 32 * li + 16 * H);
+    h8 ab, sb;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        ab[2 * j] = static_cast<_Float16>(static_cast<int16_t>(bv[j] & 0xFFFF));
+        ab[2 * j + 1] = static_cast<_Float16>(static_cast<int16_t>(bv[j] >> 16));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        sb[j] = static_cast<_Float16>(static_cast<int8_t>((sc[2 * H + j / 4] >> (8 * (j % 4))) & 0xFF));
+    }
+    const f16v cf = mfma32(ab, sb, f16v{});
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t rq = 8 * q + 4 * H;
+        const f4 yd = *reinterpret_cast<const f4*>(S + D + 4 * rq);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = 4 * q + k;
+            acc[i] += (wd * yd[k]) * (static_cast<float>(isum[i]) - 32.0f * cf[i]);
+        }
+    }
+}
+
+template <uint32_t T>
+struct ks_layout {
+    static constexpr bool k = T == qtype_q4_k || T == qtype_q6_k;
+    static constexpr uint32_t win = T == qtype_q4_k ? 144 : (T == qtype_q6_k ? k6_win : k32_wwin<T>);  // a weight row's
+    static constexpr uint32_t a = 32 * win;                       // activation qs or windows
+    static constexpr uint32_t bs = a + 32 * (k ? 256 : k32_awin);  // sums of 16 (k only)
+    static constexpr uint32_t d = bs + (k ? 1024 : 0);            // scales
+    static constexpr uint32_t stage = d + 256;
+    static constexpr uint32_t wch = win / 16;                     // 16-byte chunks
+    static constexpr int wcopies = (32 * wch + 63) / 64;
+    static constexpr int acopies = k ? 8 : (32 * 5 + 63) / 64;
+    static constexpr int copies = wcopies + acopies + (k ? 2 : 0);
+    static constexpr int stages = k ? 2 : 3;
+    static constexpr uint32_t unit_w = k ? block_bytes<T> : 2 * block_bytes<T>;  // bytes of a unit in a weight row
+    static constexpr uint32_t unit_a = k ? 292 : 68;                             //   and in an activation row
+};
+
+template <uint32_t T>
+__global__ __launch_bounds__(256) void gemm_ks_kernel(const uint8_t* w, const uint8_t* act, const float* bias,
+                                                      float* out, uint32_t n, uint32_t rows, uint32_t cols,
+                                                      uint32_t act_tiles) {
+    using L = ks_layout<T>;
+    constexpr uint32_t WAVE = L::stages * L::stage;
+    static_assert(4 * WAVE >= 4 * 16 * 256, "the merge does not fit the stages");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[4 * WAVE];
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t ln = tid & 63, H = ln >> 5, li = ln & 31;
+    const uint32_t units = cols / (L::k ? 256 : 64);
+    const uint32_t wrow = units * L::unit_w, arow = units * L::unit_a;
+    // Blocks go to the 8 XCDs in turn; each takes a contiguous run of tiles,
+    // the activation tiles of one weight tile next to each other.
+    const uint32_t total = gridDim.x, xcd = blockIdx.x % 8;
+    const uint32_t id = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+    const uint32_t o0 = id / act_tiles * 32, t0 = id % act_tiles * 32;
+
+    // Rows past the last read zeros. Whole dwords: a copy's range check is
+    // per dword, and the last row may end inside one.
+    const uint8_t* wp = w + static_cast<std::size_t>(o0) * wrow;
+    const uint32_t delta = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wp) & 3);
+    const uint8_t* wbase = wp - delta;
+    const uint32_t wbytes = (min(32u, rows - o0) * wrow + delta + 3) & ~3u;
+    const uint8_t* abase = act + static_cast<std::size_t>(t0) * arow;
+    const uint32_t abytes = min(32u, n - t0) * arow;
+
+    // A Q6_K unit U starts at byte delta + row wrow + 210 U: its window starts
+    // at the dword at or before (U = wv mod 4 fixes the parity of U).
+    const uint32_t odd = T == qtype_q6_k ? 2 * (wv & 1) : 0;
+    uint32_t wo[L::wcopies], ao[L::acopies];
+#pragma unroll
+    for (int i = 0; i < L::wcopies; ++i) {
+        const uint32_t ch = 64 * i + ln, r = ch / L::wch;
+        const uint32_t at = delta + r * wrow + odd;
+        wo[i] = r < 32 ? (T == qtype_q6_k ? at & ~3u : at) + 16 * (ch % L::wch) : buffer_oob;
+    }
+#pragma unroll
+    for (int i = 0; i < L::acopies; ++i) {
+        if constexpr (L::k) {
+            const uint32_t row = 4 * i + (ln >> 4);
+            ao[i] = row * arow + 4 + 16 * ((ln & 15) ^ (row & 15));
+        } else {
+            const uint32_t ch = 64 * i + ln;
+            ao[i] = ch < 160 ? ch / 5 * arow + 16 * (ch % 5) : buffer_oob;
+        }
+    }
+    const uint32_t bo = (ln >> 1) * arow + 260 + 16 * (ln & 1);
+    const uint32_t dof = ln < 32 ? ln * arow : buffer_oob;
+
+    uint8_t* const mine = lds + wv * WAVE;
+    const uint32_t L0 = __builtin_amdgcn_readfirstlane(lds_address(mine));
+    const auto issue = [&](uint32_t U, uint32_t slot) __attribute__((always_inline)) {
+        // (a unit past the last copies zeros, without a request)
+        const uint32_t S = L0 + slot * L::stage;
+        const uint32_t shift = U < units ? U * L::unit_w - odd : 0;
+        const rsrc wr = make_rsrc(wbase + shift, U < units ? wbytes - shift : 0);
+        const rsrc ar = make_rsrc(abase + (U < units ? U * L::unit_a : 0), U < units ? abytes - U * L::unit_a : 0);
+#pragma unroll
+        for (int i = 0; i < L::wcopies; ++i) {
+            if (64 * i + 64 <= 32 * L::wch || ln < 32 * L::wch - 64 * i) {
+                copy16_lds(wr, S + 1024 * i, wo[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < L::acopies; ++i) {
+            if (L::k || 64 * i + 64 <= 160 || ln < 160 - 64 * i) {
+                copy16_lds(ar, S + L::a + 1024 * i, ao[i]);
+            }
+        }
+        if constexpr (L::k) {
+            copy16_lds(ar, S + L::bs, bo);
+            copy4_lds(ar, S + L::d, dof);
+        }
+    };
+
+    float acc[1][16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        acc[0][i] = 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < L::stages - 1; ++i) {
+        issue(wv + 4 * i, i);
+    }
+    uint32_t slot = 0, free = L::stages - 1;
+    for (uint32_t U = wv; U < units; U += 4) {
+        // The slot the copies take was read in the step before: its reads are
+        // done (their results were used; the wait makes sure).
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue(U + 4 * (L::stages - 1), free);
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(L::copies * (L::stages - 1)) : "memory");
+        const uint8_t* S = mine + slot * L::stage;
+        if constexpr (T == qtype_q4_k) {
+            k4_block<L::a, L::bs, L::d>(S, S + li * 144, H, li, acc[0]);
+        } else if constexpr (T == qtype_q6_k) {
+            k6_block<L::a, L::bs, L::d>(S, S + li * k6_win, (delta + li * wrow + odd) & 3, H, li, acc[0]);
+        } else {
+            // d_a of row li, block H, from the row's window.
+            float* da = reinterpret_cast<float*>(mine + slot * L::stage + L::d);
+            da[ln] = half_bits(*reinterpret_cast<const uint16_t*>(S + L::a + li * k32_awin + 34 * H));
+            k32_block<T, 0, 1>(S + li * L::win, S + L::a, da, H, li, acc);
+            k32_block<T, 1, 1>(S + li * L::win, S + L::a, da, H, li, acc);
+        }
+        slot = slot + 1 == L::stages ? 0 : slot + 1;
+        free = free + 1 == L::stages ? 0 : free + 1;
+    }
+    // The empty copies behind the last unit land before the stages are reused.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+
+    // ---- the four waves' sums, in order; wave v writes rows 8 v .. 8 v + 7 -----------------
+    f4* part = reinterpret_cast<f4*>(lds);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        part[(wv * 4 + q) * 64 + ln] = f4{acc[0][4 * q], acc[0][4 * q + 1], acc[0][4 * q + 2], acc[0][4 * q + 3]};
+    }
+    lds_barrier();
+    f4 sum = part[wv * 64 + ln];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) {
+        const f4 p = part[(v * 4 + wv) * 64 + ln];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            sum[i] += p[i];
+        }
+    }
+    const uint32_t o = o0 + li;
+    if (o < rows) {
+        const float bo2 = bias != nullptr ? bias[o] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t r = t0 + 8 * wv + 4 * H + i;
+            if (r < n) {
+                out[static_cast<std::size_t>(r) * rows + o] = bias != nullptr ? sum[i] + bo2 : sum[i];
+            }
+        }
+    }
+}
+
+// ---- a few activation rows: 16-row tiles ------------------------------------------------
+//
+// Up to 32 activation rows: weights pass once, so what counts is to keep every
+// CU reading them and to decode each weight once. A block owns 16 weight rows
+// (a 4096-row product is 256 blocks, one per CU) and its eight waves every
+// eighth 256 columns; v_mfma_i32_16x16x64_i8 gives a lane the 16 columns of
+// one Q6_K sub-block (or half of one of Q4_K's), so a scale is one value per
+// lane. Q6_K's scales are folded into the weights here: w = sc (q - 32) lies
+// within +-4096, and w = 256 h + l with int8 h and l makes two products that
+// accumulate in place over the whole block, exact integers as before, in
+// place of one product and 16 multiply-adds per sub-block. (Lane group G takes
+// sub-blocks 8 (G / 2) + 2 j + G % 2 in product j: those share its qh bytes,
+// and a lane decodes 64 weights from 48 bytes read once.)
+//
+// A wave stages 256 columns of its rows in its own LDS, reads all operands
+// into registers, sends the next copies off and only then decodes and
+// multiplies: one stage, no barrier. The eight partial sums meet in a fixed
+// order. 24 rows against Q6_K 4096 x 14336: 22 us a call with the quantizer
+// (48 MB of weights, 2.2 TB/s), 147 us as six passes of the GEMV; bound by
+// the decode (about 300 vector instructions per 16 x 256 weights) and, above
+// 16 rows, one block per CU for its LDS.
+
+template <uint32_t T>
+struct r16_layout {
+    static constexpr bool k = T == qtype_q4_k || T == qtype_q6_k;
+    static constexpr uint32_t unit_w = k ? block_bytes<T> : 8 * block_bytes<T>;  // 256 columns of a weight row
+    static constexpr uint32_t unit_a = k ? 292 : 272;                            //   and of an activation row
+    // A weight row's window in LDS, whole 16-byte chunks 4 (mod 8) dwords apart
+    // or so, for the banks: 144, 240; 272, 144, 176.
+    static constexpr uint32_t win = T == qtype_q6_k ? k6_win : unit_w;
+    static constexpr uint32_t wch = win / 16;
+};
+
+template <uint32_t T, int AT>
+struct r16_stage {
+    using L = r16_layout<T>;
+    static constexpr uint32_t a = 16 * L::win;                         // activation qs (k) or windows
+    static constexpr uint32_t bs = a + 16 * AT * (L::k ? 256 : 272);   // sums of 16 (k only)
+    static constexpr uint32_t d = bs + (L::k ? 512 * AT : 0);          // scales, f32
+    static constexpr uint32_t bytes = d + (L::k ? 256 : 8 * 16 * AT * 4);
+};
+
+template <uint32_t T, int AT>
+__global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const uint8_t* act, const float* bias,
+                                                       float* out, uint32_t n, uint32_t rows, uint32_t cols) {
+    using L = r16_layout<T>;
+    using ST = r16_stage<T, AT>;
+    constexpr uint32_t NW = 8, AR = 16 * AT;
+    static_assert(ST::bytes % 16 == 0 && ST::bytes >= AT * 4 * 256, "stage layout");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[NW * ST::bytes];
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t ln = tid & 63, G = ln >> 4, c = ln & 15;
+    const uint32_t units = (cols + 255) / 256;  // (the last may be partial for the 32-block formats)
+    const uint32_t wrow = L::k ? units * L::unit_w : cols / 32 * block_bytes<T>;
+    const uint32_t arow = L::k ? units * L::unit_a : cols / 32 * 34;
+    const uint32_t o0 = blockIdx.x * 16;
+
+    const uint8_t* wp = w + static_cast<std::size_t>(o0) * wrow;
+    const uint32_t delta = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wp) & 3);
+    const uint8_t* wbase = wp - delta;
+    // Rows past the last read zeros. Whole dwords: a copy's range check is
+    // per dword, and the last row may end inside one.
+    const uint32_t wbytes = (min(16u, rows - o0) * wrow + delta + 3) & ~3u;
+    const uint8_t* abase = act;
+    const uint32_t abytes = n * arow;  // (n <= AR; rows past it read zeros)
+
+    // Copies: chunk ch = 64 i + ln of the 16 weight row windows, then the
+    // activation rows' (k: qs with chunk x in slot x ^ (row % 16), bsums, d;
+    // else windows of 17 chunks). A Q6_K unit U starts at byte delta + row
+    // wrow + 210 U, its window at the dword at or before (U = wv mod 8 fixes
+    // the parity of U).
+    constexpr int WC = (16 * L::wch + 63) / 64, ACH = L::k ? 16 : 17, AC = (AR * ACH + 63) / 64;
+    const uint32_t odd = T == qtype_q6_k ? 2 * (wv & 1) : 0;
+    uint32_t wo[WC], ao[AC];
+#pragma unroll
+    for (int i = 0; i < WC; ++i) {
+        const uint32_t ch = 64 * i + ln, r = ch / L::wch, at = delta + r * wrow + odd;
+        wo[i] = (T == qtype_q6_k ? at & ~3u : at) + 16 * (ch % L::wch);
+    }
+#pragma unroll
+    for (int i = 0; i < AC; ++i) {
+        const uint32_t ch = 64 * i + ln, r = ch / ACH, x = ch % ACH;
+        ao[i] = L::k ? r * arow + 4 + 16 * (x ^ (r & 15)) : r * arow + 16 * x;
+    }
+    const uint32_t bo = (ln >> 1) * arow + 260 + 16 * (ln & 1);
+    const uint32_t dof = ln * arow;
+
+    uint8_t* const S = lds + wv * ST::bytes;
+    const uint32_t L0 = __builtin_amdgcn_readfirstlane(lds_address(S));
+    const auto issue = [&](uint32_t U) __attribute__((always_inline)) {
+        const uint32_t shift = U * L::unit_w - odd;
+        const rsrc wr = make_rsrc(wbase + shift, wbytes - shift);
+        const rsrc ar = make_rsrc(abase + U * L::unit_a, abytes - U * L::unit_a);
+#pragma unroll
+        for (int i = 0; i < WC; ++i) {
+            if (64 * i + 64 <= 16 * L::wch || ln < 16 * L::wch - 64 * i) {
+                copy16_lds(wr, L0 + 1024 * i, wo[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < AC; ++i) {
+            if (64 * i + 64 <= AR * ACH || ln < AR * ACH - 64 * i) {
+                copy16_lds(ar, L0 + ST::a + 1024 * i, ao[i]);
+            }
+        }
+        if constexpr (L::k) {
+            if (T == qtype_q4_k && ln < 2 * AR) {
+                copy16_lds(ar, L0 + ST::bs, bo);
+            }
+            if (ln < AR) {
+                copy4_lds(ar, L0 + ST::d, dof);
+            }
+        }
+    };
+
+    f4 acc[AT];
+#pragma unroll
+    for (int t = 0; t < AT; ++t) {
+        acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const auto mma = [](const u4& a, const u4& b, i4v d) __attribute__((always_inline)) {
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i4v, a), __builtin_bit_cast(i4v, b), d, 0, 0, 0);
+    };
+    if (wv < units) {
+        issue(wv);
+    }
+    for (uint32_t U = wv; U < units; U += NW) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (T == qtype_q6_k) {
+            const uint8_t* RB = S + c * k6_win;
+            const uint32_t o = (delta + c * wrow + odd) & 3, hf = G >> 1, e = G & 1;
+            // 16 bytes at byte b (a multiple of 16) of the block.
+            const auto chunk = [&](uint32_t b) __attribute__((always_inline)) {
+                const u4 x = *reinterpret_cast<const u4*>(RB + b);
+                const uint32_t y = *reinterpret_cast<const uint32_t*>(RB + b + 16);
+                return u4{__builtin_amdgcn_alignbyte(x[1], x[0], o), __builtin_amdgcn_alignbyte(x[2], x[1], o),
+                          __builtin_amdgcn_alignbyte(x[3], x[2], o), __builtin_amdgcn_alignbyte(y, x[3], o)};
+            };
+            const u4 ql[2] = {chunk(64 * hf + 16 * e), chunk(64 * hf + 32 + 16 * e)};
+            const u4 qh = chunk(128 + 32 * hf + 16 * e);
+            const u4 sc4 = chunk(192);
+            const uint32_t dd = __builtin_amdgcn_alignbyte(*reinterpret_cast<const uint32_t*>(RB + 212),
+                                                           *reinterpret_cast<const uint32_t*>(RB + 208), o);
+            const float wd = half_bits(dd & 0xFFFF);
+            u4 a[AT][4];
+            f4 yd[AT];
+#pragma unroll
+            for (int t = 0; t < AT; ++t) {
+                yd[t] = *reinterpret_cast<const f4*>(S + ST::d + 64 * t + 16 * G);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    a[t][j] = *reinterpret_cast<const u4*>(S + ST::a + (16 * t + c) * 256 + 16 * ((8 * hf + 2 * j + e) ^ c));
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (U + NW < units) {
+                issue(U + NW);
+            }
+            // Scales 8 hf + 2 j + e: bytes e and 2 + e of two dwords.
+            const uint32_t s01 = hf ? sc4[2] : sc4[0], s23 = hf ? sc4[3] : sc4[1];
+            i4v lo[AT] = {}, hi[AT] = {};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int sc = static_cast<int8_t>(((j < 2 ? s01 : s23) >> (16 * (j & 1) + 8 * e)) & 0xFF);
+                const uint32_t scp = (static_cast<uint32_t>(sc) & 0xFFFF) * 0x10001u;
+                const uint32_t add = (static_cast<uint32_t>(128 - 32 * sc) & 0xFFFF) * 0x10001u;
+                u4 pl, ph;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const uint32_t l4 = (ql[j & 1][x] >> (4 * (j >> 1))) & 0x0F0F0F0Fu;
+                    const uint32_t h2 = (j < 2 ? qh[x] << (4 - 2 * j) : qh[x] >> (2 * j - 4)) & 0x30303030u;
+                    const uint32_t q = l4 | h2;
+                    // sc (q - 32) + 128 of bytes 0, 2 and 1, 3, in 16 bits.
+                    const auto mad = [&](uint32_t v) {
+                        return __builtin_bit_cast(uint32_t, static_cast<u16x2>(__builtin_bit_cast(u16x2, v) *
+                                                                               __builtin_bit_cast(u16x2, scp) +
+                                                                               __builtin_bit_cast(u16x2, add)));
+                    };
+                    const uint32_t we = mad(q & 0x00FF00FFu), wo2 = mad((q >> 8) & 0x00FF00FFu);
+                    pl[x] = __builtin_amdgcn_perm(wo2, we, 0x06020400u) ^ 0x80808080u;
+                    ph[x] = __builtin_amdgcn_perm(wo2, we, 0x07030501u);
+                }
+#pragma unroll
+                for (int t = 0; t < AT; ++t) {
+                    lo[t] = mma(a[t][j], pl, lo[t]);
+                    hi[t] = mma(a[t][j], ph, hi[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < AT; ++t) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    acc[t][r] += (wd * yd[t][r]) * static_cast<float>(lo[t][r] + (hi[t][r] << 8));
+                }
+            }
+        } else if constexpr (T == qtype_q4_k) {
+            const uint8_t* Wl = S + c * 144;
+            const u4 hdr = *reinterpret_cast<const u4*>(Wl);
+            // Product j: sub-blocks 2 j (lane groups 0, 1) and 2 j + 1 (2, 3),
+            // halves G % 2: the low and high nibbles of 16 bytes.
+            u4 qw[4], a[AT][4], bv[AT];
+            f4 yd[AT];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                qw[j] = *reinterpret_cast<const u4*>(Wl + 16 + 32 * j + 16 * (G & 1));
+            }
+#pragma unroll
+            for (int t = 0; t < AT; ++t) {
+                yd[t] = *reinterpret_cast<const f4*>(S + ST::d + 64 * t + 16 * G);
+                bv[t] = *reinterpret_cast<const u4*>(S + ST::bs + 32 * (16 * t + c) + 16 * (G & 1));
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    a[t][j] = *reinterpret_cast<const u4*>(S + ST::a + (16 * t + c) * 256 + 16 * ((4 * j + G) ^ c));
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (U + NW < units) {
+                issue(U + NW);
+            }
+            const float wd = half_bits(hdr[0] & 0xFFFF), wdmin = half_bits(hdr[0] >> 16);
+            const uint32_t sc[2] = {hdr[1] & 0x3F3F3F3Fu, (hdr[3] & 0x0F0F0F0Fu) | ((hdr[1] >> 2) & 0x30303030u)};
+            const uint32_t mn[2] = {hdr[2] & 0x3F3F3F3Fu,
+                                    ((hdr[3] >> 4) & 0x0F0F0F0Fu) | ((hdr[2] >> 2) & 0x30303030u)};
+            const uint32_t e = G >> 1;  // nibble, sub-block parity
+            i4v lo[AT] = {}, hi[AT] = {};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t sj = (sc[j / 2] >> (8 * (2 * j % 4) + 8 * e)) & 0xFF;
+                const uint32_t sl = (sj & 7) * 0x10001u, sh = (sj >> 3) * 0x10001u;
+                u4 pl, ph;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const uint32_t nib = (qw[j][x] >> (4 * e)) & 0x0F0F0F0Fu;
+                    pl[x] = mul_u16x2(nib, sl);
+                    ph[x] = mul_u16x2(nib, sh);
+                }
+#pragma unroll
+                for (int t = 0; t < AT; ++t) {
+                    lo[t] = mma(a[t][j], pl, lo[t]);
+                    hi[t] = mma(a[t][j], ph, hi[t]);
+                }
+            }
+            // mins: the 16 activation sums (lane groups 0, 1; zero above)
+            // against m of their sub-block, as in k4_block.
+            h8 mb;
+            const uint32_t mh = mn[G & 1];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const _Float16 m = G < 2 ? static_cast<_Float16>(static_cast<float>((mh >> (8 * j)) & 0xFF))
+                                         : static_cast<_Float16>(0.0f);
+                mb[2 * j] = m;
+                mb[2 * j + 1] = m;
+            }
+#pragma unroll
+            for (int t = 0; t < AT; ++t) {
+                h8 ab;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    ab[2 * j] = static_cast<_Float16>(static_cast<int16_t>(bv[t][j] & 0xFFFF));
+                    ab[2 * j + 1] = static_cast<_Float16>(static_cast<int16_t>(bv[t][j] >> 16));
+                }
+                const f4 fm = mfma16(ab, mb, f4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int isum = lo[t][r] + (hi[t][r] << 3);
+                    acc[t][r] += yd[t][r] * (wd * static_cast<float>(isum) - wdmin * fm[r]);
+                }
+            }
+        } else {
+            // Blocks of 32: v_mfma_i32_16x16x32_i8, lane group G columns 8 G
+            // .. 8 G + 7. The activation scales go to LDS as f32 [block][row].
+            const uint32_t nblk = min(8u, cols / 32 - 8 * U);
+            float* da = reinterpret_cast<float*>(S + ST::d);
+#pragma unroll
+            for (uint32_t i = 0; i < 8 * AR / 64; ++i) {
+                const uint32_t x = 64 * i + ln, r = x % AR, b = x / AR;
+                da[x] = half_bits(*reinterpret_cast<const uint16_t*>(S + ST::a + r * 272 + 34 * b));
+            }
+            // N dwords from byte at (even) of p (4-aligned).
+            const auto words = [&]<int N>(const uint8_t* p, uint32_t at, uint32_t (&d)[N]) __attribute__((always_inline)) {
+                const uint32_t* x = reinterpret_cast<const uint32_t*>(p + (at & ~3u));
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    d[i] = (at & 3) ? __builtin_amdgcn_alignbyte(x[i + 1], x[i], 2) : x[i];
+                }
+            };
+            const uint8_t* WR = S + c * L::win;
+            const auto block = [&]<int b>() __attribute__((always_inline)) {
+                constexpr uint32_t B = b * block_bytes<T>;
+                const float dw = half_bits(*reinterpret_cast<const uint16_t*>(WR + B));
+                uint32_t q[2];
+                if constexpr (T == qtype_q8_0) {
+                    words(WR + 8 * G, B + 2, q);
+                } else {
+                    constexpr uint32_t Q = B + (T == qtype_q5_0 ? 6 : 2);
+                    uint32_t qs[2];
+                    words(WR + 8 * (G & 1), Q, qs);
+                    if constexpr (T == qtype_q4_0) {
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            q[i] = sext4((qs[i] >> (4 * (G >> 1))) & 0x0F0F0F0Fu);
+                        }
+                    } else {
+                        uint32_t hb[1];
+                        words(WR, B + 2, hb);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            q[i] = sext5(((qs[i] >> (4 * (G >> 1))) & 0x0F0F0F0Fu) |
+                                         spread4((hb[0] >> (8 * G + 4 * i)) & 0xF));
+                        }
+                    }
+                }
+                const long bw = static_cast<long>((static_cast<uint64_t>(q[1]) << 32) | q[0]);
+#pragma unroll
+                for (int t = 0; t < AT; ++t) {
+                    uint32_t av[2];
+                    words(S + ST::a + (16 * t + c) * 272 + 8 * G, 34 * b + 2, av);
+                    const long a = static_cast<long>((static_cast<uint64_t>(av[1]) << 32) | av[0]);
+                    const i4v cm = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bw, i4v{}, 0, 0, 0);
+                    const f4 d4 = *reinterpret_cast<const f4*>(da + AR * b + 16 * t + 4 * G);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[t][r] += static_cast<float>(cm[r]) * (dw * d4[r]);
+                    }
+                }
+            };
+            const auto part = [&]<int b>() __attribute__((always_inline)) {
+                if (b < nblk) {  // wave-uniform
+                    block.template operator()<b>();
+                }
+            };
+            block.template operator()<0>();
+            block.template operator()<1>();
+            part.template operator()<2>();
+            part.template operator()<3>();
+            part.template operator()<4>();
+            part.template operator()<5>();
+            part.template operator()<6>();
+            part.template operator()<7>();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (U + NW < units) {
+                issue(U + NW);
+            }
+        }
+    }
+
+    // ---- the eight waves' sums, in order: wave v adds tile v's ------------------------------
+    lds_barrier();
+    f4* part = reinterpret_cast<f4*>(lds);
+#pragma unroll
+    for (int t = 0; t < AT; ++t) {
+        part[(wv * AT + t) * 64 + ln] = acc[t];
+    }
+    lds_barrier();
+    if (wv >= AT) {
+        return;
+    }
+    f4 sum = part[wv * 64 + ln];
+#pragma unroll
+    for (uint32_t v = 1; v < NW; ++v) {
+        const f4 p = part[(v * AT + wv) * 64 + ln];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            sum[r] += p[r];
+        }
+    }
+    const uint32_t o = o0 + c;
+    if (o < rows) {
+        const float bo2 = bias != nullptr ? bias[o] : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t row = 16 * wv + 4 * G + r;
+            if (row < n) {
+                out[static_cast<std::size_t>(row) * rows + o] = bias != nullptr ? sum[r] + bo2 : sum[r];
+            }
+        }
+    }
+}
 }  // namespace
+
+namespace {
+
+// The 32-block formats' staged kernels copy row windows of whole blocks: every
+// unit of two blocks starts on a dword when cols is a multiple of 64 (w and
+// act are 4-byte aligned, as the interface keeps them).
+bool staged_ok(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t cols) {
+    return t == qtype_q4_k || t == qtype_q6_k ||
+           (cols % 64 == 0 && (reinterpret_cast<uintptr_t>(w) & 3) == 0 && (reinterpret_cast<uintptr_t>(act) & 3) == 0);
+}
+
+// Calls go.operator()<T>() for the weight type.
+template <class F>
+void for_qtype(uint32_t t, const F& go) {
+    switch (t) {
+    case qtype_q4_0:
+        go.template operator()<qtype_q4_0>();
+        break;
+    case qtype_q5_0:
+        go.template operator()<qtype_q5_0>();
+        break;
+    case qtype_q8_0:
+        go.template operator()<qtype_q8_0>();
+        break;
+    case qtype_q4_k:
+        go.template operator()<qtype_q4_k>();
+        break;
+    default:
+        go.template operator()<qtype_q6_k>();
+        break;
+    }
+}
+
+}  // namespace
+
+// The GEMV passes over the weights once per four activation rows and decodes
+// them on the way for each; a matrix-core tile takes 16. us per call (4096 x
+// 14336, 14336 x 4096, 4096 x 4096 weights), GEMV against 16-row tiles: Q4_K
+// 2 rows 16.8 / 12.8, 14.3 / 13.6, 7.9 / 7.9; Q6_K 19.3 / 16.7, 16.5 / 17.8,
+// 9.3 / 9.0; Q8_0 22.7 / 18.9, 16.9 / 19.5, 11.0 / 9.3: even at two rows; at
+// four Q4_K 23.7 / 12.8, 22.6 / 14.3, 12.2 / 8.3.
+bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t cols) {
+    return n >= (staged_ok(t, w, act, cols) ? 3u : 32u);
+}
 
 hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
                          uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream) {
@@ -914,41 +1689,51 @@ hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* 
     } else {
         quantize_act_kernel<false><<<qblocks, 256, 0, stream>>>(x, act, n, cols);
     }
-    const dim3 grid((rows + gq_m - 1) / gq_m, (n + gq_n - 1) / gq_n);
-    // The 32-block formats through LDS when every row's stage starts on a
-    // dword (whole stages of two blocks; w and act 4-byte aligned, as the
-    // interface keeps them); else the register kernel.
-    const bool staged = cols % 64 == 0 && (reinterpret_cast<uintptr_t>(w) & 3) == 0 &&
-                        (reinterpret_cast<uintptr_t>(act) & 3) == 0;
-    switch (t) {
-    case qtype_q4_0:
-        if (staged) {
-            gemm_qb32_kernel<qtype_q4_0><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        } else {
-            gemm_q_kernel<qtype_q4_0><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        }
-        break;
-    case qtype_q5_0:
-        if (staged) {
-            gemm_qb32_kernel<qtype_q5_0><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        } else {
-            gemm_q_kernel<qtype_q5_0><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        }
-        break;
-    case qtype_q8_0:
-        if (staged) {
-            gemm_qb32_kernel<qtype_q8_0><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        } else {
-            gemm_q_kernel<qtype_q8_0><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        }
-        break;
-    case qtype_q4_k:
-        gemm_q4k_kernel<<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        break;
-    default:
-        gemm_q6k_kernel<<<dim3((rows + 63) / 64, grid.y), 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
-        break;
+    const bool staged = staged_ok(t, w, act, cols);
+    // Up to 32 rows: 16-row weight tiles, the weights read once. us per call
+    // at 24 rows, GEMV passes against these tiles: Q6_K 4096 x 14336 147 /
+    // 22, 14336 x 4096 112 / 29; Q4_K 112 / 18, 110 / 23; Q8_0 133 / 27, 90 /
+    // 33; 1024 x 4096 30 / 9 (Q4_K).
+    if (staged && n <= 32) {
+        const uint32_t tiles = (rows + 15) / 16;
+        for_qtype(t, [&]<uint32_t T>() {
+            if (n <= 16) {
+                gemm_r16_kernel<T, 1><<<tiles, 512, 0, stream>>>(w, act, bias, out, n, rows, cols);
+            } else {
+                gemm_r16_kernel<T, 2><<<tiles, 512, 0, stream>>>(w, act, bias, out, n, rows, cols);
+            }
+        });
+        return hipGetLastError();
     }
+    // While a product is few tiles of 32 x 32, those with the columns split
+    // over the waves; beyond, the larger tiles decode a weight for more
+    // activation rows. us per call, larger tiles against these: Q4_K 4096 x
+    // 14336 at 64 rows 93 / 23, at 256 (1024 tiles) 98 / 72, at 512 107 / 136;
+    // 14336 x 4096 at 64 (896) 35 / 30, at 128 37 / 47; Q6_K 4096 x 4096 at
+    // 256 (1024) 51 / 44, at 512 67 / 81. The 32-block formats, two blocks to
+    // a CU and slower in the larger tiles: Q8_0 4096 x 14336 at 512 (2048
+    // tiles) 244 / 212, 14336 x 4096 at 128 (1792) 78 / 65, at 256 93 / 114.
+    const uint32_t act_tiles = (n + 31) / 32;
+    const uint64_t tiles = uint64_t{(rows + 31) / 32} * act_tiles;
+    if (staged && tiles <= (kq ? 1024u : 2048u)) {
+        for_qtype(t, [&]<uint32_t T>() {
+            gemm_ks_kernel<T><<<static_cast<uint32_t>(tiles), 256, 0, stream>>>(w, act, bias, out, n, rows, cols,
+                                                                                act_tiles);
+        });
+        return hipGetLastError();
+    }
+    const dim3 grid((rows + gq_m - 1) / gq_m, (n + gq_n - 1) / gq_n);
+    for_qtype(t, [&]<uint32_t T>() {
+        if constexpr (T == qtype_q4_k) {
+            gemm_q4k_kernel<<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
+        } else if constexpr (T == qtype_q6_k) {
+            gemm_q6k_kernel<<<dim3((rows + 63) / 64, grid.y), 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
+        } else if (staged) {
+            gemm_qb32_kernel<T><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
+        } else {
+            gemm_q_kernel<T><<<grid, 256, 0, stream>>>(w, act, bias, out, n, rows, cols);
+        }
+    });
     return hipGetLastError();
 }
 

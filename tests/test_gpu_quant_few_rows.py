@@ -1,0 +1,97 @@
+"""GPU parity of quantized products with few activation rows or few tiles: the
+matrix-core kernels whose waves split the columns (gemm_r16_kernel up to 32
+rows, gemm_ks_kernel above), at the edges of their tiles, units and rules."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import quant_host as qh
+from gpu_util import Arena
+from synapse_amd.gguf import BLOCK, Q4_0, Q4_K, Q5_0, Q6_K, Q8_0
+from test_gpu_quant import matmul_q, random_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def arena():
+    a = Arena(256 << 20)
+    yield a
+    a.close()
+
+
+# Rows: the last GEMV (2) and the first tile (3), one and two tiles of 16
+# activation rows whole and cut, then 32 x 32 tiles (33 on). Weight rows: one,
+# a tile less one, whole and one over; odd counts start rows off a dword
+# (Q6_K). Columns: one unit (seven waves idle), one per wave, one more, and
+# for the 32-block formats a last unit of two to six blocks, and one of 25
+# blocks (odd: the kernels that copy whole units do not take it).
+CASES = [(2, 17, 512), (3, 1, 256), (3, 15, 2048), (5, 33, 2304), (15, 16, 768), (16, 31, 4096), (17, 16, 256),
+         (24, 65, 14336), (31, 5, 2560), (32, 130, 1024), (33, 31, 256), (40, 33, 1280), (64, 65, 1024), (65, 32, 2048),
+         (96, 7, 768), (3, 17, 64), (16, 15, 320), (20, 33, 448), (33, 9, 64), (40, 33, 192), (31, 20, 800),
+         (33, 20, 800)]
+
+
+@pytest.mark.parametrize("t", [Q4_0, Q5_0, Q8_0, Q4_K, Q6_K])
+@pytest.mark.parametrize("n,rows,cols", CASES)
+def test_few_rows(arena, t, n, rows, cols):
+    """Activation bytes are ggml's bit for bit; every output is within 1e-5 of
+    sum |w| |x^| of the exact product (the block integers are exact: at most
+    cols / 32 + 10 float combines, each of 3 roundings of 6e-8)."""
+    if cols % BLOCK[t][0]:
+        pytest.skip("cols not whole blocks")
+    _check(arena, t, n, rows, cols)
+
+
+# The last count of 32 x 32 tiles that gemm_ks_kernel takes, and one row more.
+@pytest.mark.parametrize("t,rows,cols", [(Q4_K, 16384, 256), (Q4_K, 16385, 256), (Q6_K, 16384, 256), (Q6_K, 16385, 256),
+                                         (Q8_0, 32768, 64), (Q8_0, 32769, 64)])
+def test_tile_count_rule(arena, t, rows, cols):
+    _check(arena, t, 33, rows, cols)
+
+
+def _check(arena, t, n, rows, cols):
+    rng = np.random.default_rng(100000 * t + 1000 * n + rows + cols)
+    raw = random_blocks(t, rows, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[1, :64] = 0.0
+    if n > 2:
+        x[2] = 0.0  # zero blocks only
+    bias = rng.standard_normal(rows).astype(np.float32)
+    want_act = np.concatenate([qh.quantize_act(x[r], t) for r in range(n)])
+    w = qh.dequantize(raw, t).reshape(rows, cols).astype(np.float64)
+    xa = np.stack([qh.dequantize_act(a, qh.act_type(t)) for a in want_act.reshape(n, -1)]).astype(np.float64)
+    exact, scale = xa @ w.T, np.abs(xa) @ np.abs(w).T
+    for b in (None, bias):
+        out, act = matmul_q(arena, raw, t, x, rows, cols, b) if b is not None else matmul_q(arena, raw, t, x, rows, cols)
+        assert np.array_equal(act, want_act)
+        got = out.astype(np.float64) - (0 if b is None else b)
+        err = np.abs(got - exact)
+        assert np.all(err <= 1e-5 * np.maximum(scale, 1.0)), float((err / np.maximum(scale, 1.0)).max())
+
+
+@pytest.mark.parametrize("n", [24, 48])
+def test_extreme_weights(arena, n):
+    """Q6_K and Q4_K blocks whose quants and scales sit at the ends of their
+    ranges against activations at +-127: the largest integers the folded
+    weight planes and their sums can reach."""
+    rows, cols = 32, 512
+    rng = np.random.default_rng(n)
+    for t in (Q6_K, Q4_K):
+        blocks = random_blocks(t, rows, cols, rng).reshape(rows * cols // 256, -1)
+        for i, blk in enumerate(blocks):
+            if t == Q6_K:
+                blk[:192] = 0xFF if i % 2 else 0x00     # q = 63 or 0
+                blk[192:208] = 0x80 if i % 3 else 0x7F  # scale -128 or 127
+            else:
+                blk[4:] = 0xFF  # scale, min and quants all ones
+        x = np.where(rng.random((n, cols)) < 0.5, -1.0, 1.0).astype(np.float32)
+        x[: n // 2] = np.abs(x[: n // 2])
+        raw = blocks.reshape(-1)
+        out, _ = matmul_q(arena, raw, t, x, rows, cols)
+        act = np.stack([qh.quantize_act(r, t) for r in x])
+        w = qh.dequantize(raw, t).reshape(rows, cols).astype(np.float64)
+        xa = np.stack([qh.dequantize_act(a, qh.act_type(t)) for a in act]).astype(np.float64)
+        err = np.abs(out - xa @ w.T)
+        assert np.all(err <= 1e-5 * np.maximum(np.abs(xa) @ np.abs(w).T, 1.0))
