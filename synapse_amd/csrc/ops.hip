@@ -58,6 +58,59 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* in, const fl
     }
 }
 
+// The same with the row in registers: a thread holds V chunks of four floats,
+// so the row is read once and the only waits are its loads, the wave sums and
+// one barrier (the row-loop form above: nine barriers and a second read).
+// Latency-bound at decode sizes (launch_rms_norm has the figures).
+template <int THREADS, int V>
+__global__ __launch_bounds__(THREADS) void rms_norm_vec_kernel(const float* in, const float* gamma, float* out,
+                                                               uint32_t size, float eps) {
+    constexpr int WAVES = THREADS / 64;
+    __shared__ double part[WAVES];
+    const f4* x = reinterpret_cast<const f4*>(in + static_cast<std::size_t>(blockIdx.x) * size);
+    const f4* gm = reinterpret_cast<const f4*>(gamma);
+    f4* y = reinterpret_cast<f4*>(out + static_cast<std::size_t>(blockIdx.x) * size);
+    const uint32_t chunks = size / 4;
+    f4 v[V], g[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const uint32_t i = threadIdx.x + THREADS * k;
+        v[k] = i < chunks ? x[i] : f4{0.0f, 0.0f, 0.0f, 0.0f};
+        g[k] = i < chunks ? gm[i] : f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            s += static_cast<double>(v[k][i] * v[k][i]);
+        }
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+        s += __shfl_xor(s, m, wave);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        part[threadIdx.x >> 6] = s;
+    }
+    __syncthreads();
+    double total = part[0];
+#pragma unroll
+    for (int k = 1; k < WAVES; ++k) {
+        total += part[k];
+    }
+    const float mean = static_cast<float>(total / static_cast<double>(size));
+    const float sc = 1.0f / sqrtf(mean + eps);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const uint32_t i = threadIdx.x + THREADS * k;
+        if (i < chunks) {
+            y[i] = f4{(v[k][0] * sc) * g[k][0], (v[k][1] * sc) * g[k][1], (v[k][2] * sc) * g[k][2],
+                      (v[k][3] * sc) * g[k][3]};
+        }
+    }
+}
+
 // GELU as ggml's CPU op computes it (S/kernels/elementwise.hpp:115-167):
 // x <= -10 gives 0, x >= 10 gives x; otherwise x is rounded to binary16 and
 // the tanh approximation of that half, rounded to binary16, is returned --
@@ -69,38 +122,50 @@ __device__ __forceinline__ float gelu_f16_table(float x) {
     return x <= -10.0f ? 0.0f : (x >= 10.0f ? x : t);
 }
 
-// Element-wise ops (S/kernels/elementwise.hpp:28-81).
+// One element of an element-wise op (S/kernels/elementwise.hpp:28-81).
+template <uint32_t OP>
+__device__ __forceinline__ float elementwise(float x, float b, float scalar) {
+    if constexpr (OP == elementwise_add || OP == elementwise_add_bias) {  // (kernels::add_bias on every row)
+        return x + b;
+    } else if constexpr (OP == elementwise_mul) {
+        return x * b;
+    } else if constexpr (OP == elementwise_silu_mul) {
+        // silu(x) = x / (1 + exp(-x)) rounded to float, then the product,
+        // as op_silu followed by op_mul computes it.
+        return (x / (1.0f + expf(-x))) * b;
+    } else if constexpr (OP == elementwise_gelu) {
+        return gelu_f16_table(x);
+    } else if constexpr (OP == elementwise_silu) {  // kernels::silu
+        return x / (1.0f + expf(-x));
+    } else {  // elementwise_scale
+        return x * scalar;
+    }
+}
+
+constexpr bool elementwise_reads_b(uint32_t op) {
+    return op == elementwise_add || op == elementwise_mul || op == elementwise_silu_mul || op == elementwise_add_bias;
+}
+
+// N floats per thread and trip: 4 where everything is 16-byte aligned (and b's
+// period whole chunks), else 1. Latency-bound at decode sizes: SiLU times up
+// over 14336 floats 2.4 us, an add of 4096 2.0, against 3.9 with one kernel
+// for all ops (a switch and a 64-bit remainder in its loop), one float a trip.
+template <uint32_t OP, int N>
 __global__ __launch_bounds__(256) void elementwise_kernel(const float* a, const float* b, float* out, uint64_t count,
-                                                          uint32_t op, float scalar, uint32_t period) {
-    for (uint64_t e = blockIdx.x * 256ull + threadIdx.x; e < count; e += gridDim.x * 256ull) {
-        const float x = a[e];
-        float y;
-        switch (op) {
-        case elementwise_add:
-            y = x + b[e];
-            break;
-        case elementwise_mul:
-            y = x * b[e];
-            break;
-        case elementwise_silu_mul:
-            // silu(x) = x / (1 + exp(-x)) rounded to float, then the product,
-            // as op_silu followed by op_mul computes it.
-            y = (x / (1.0f + expf(-x))) * b[e];
-            break;
-        case elementwise_gelu:
-            y = gelu_f16_table(x);
-            break;
-        case elementwise_silu:  // kernels::silu
-            y = x / (1.0f + expf(-x));
-            break;
-        case elementwise_add_bias:  // kernels::add_bias on every row
-            y = x + b[e % period];
-            break;
-        default:  // elementwise_scale
-            y = x * scalar;
-            break;
+                                                          float scalar, uint32_t period) {
+    typedef float vec __attribute__((ext_vector_type(N)));
+    const uint64_t chunks = count / N;
+    for (uint64_t e = blockIdx.x * 256ull + threadIdx.x; e < chunks; e += gridDim.x * 256ull) {
+        const vec x = reinterpret_cast<const vec*>(a)[e];
+        vec y = x;
+        if constexpr (elementwise_reads_b(OP)) {
+            y = reinterpret_cast<const vec*>(b)[OP == elementwise_add_bias ? e % (period / N) : e];
         }
-        out[e] = y;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            y[i] = elementwise<OP>(x[i], y[i], scalar);
+        }
+        reinterpret_cast<vec*>(out)[e] = y;
     }
 }
 
@@ -262,6 +327,23 @@ hipError_t launch_softmax(const float* in, float* out, uint32_t n, uint32_t size
 
 hipError_t launch_rms_norm(const float* in, const float* gamma, float* out, uint32_t n, uint32_t size, float eps,
                            hipStream_t stream) {
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    if (size % 4 == 0 && aligned(in) && aligned(gamma) && aligned(out)) {
+        // As few threads as hold the row: one row of 4096 takes 2.2 us with
+        // 256 (2.5 with 1024, 5.5 in the row-loop form), 2048 rows 10.7 (14.3,
+        // 16.9); replayed from a graph.
+        const bool held = size <= 1024 * 16;
+        if (size <= 256 * 4) {
+            rms_norm_vec_kernel<256, 1><<<n, 256, 0, stream>>>(in, gamma, out, size, eps);
+        } else if (size <= 256 * 16) {
+            rms_norm_vec_kernel<256, 4><<<n, 256, 0, stream>>>(in, gamma, out, size, eps);
+        } else if (held) {
+            rms_norm_vec_kernel<1024, 4><<<n, 1024, 0, stream>>>(in, gamma, out, size, eps);
+        }
+        if (held) {
+            return hipGetLastError();
+        }
+    }
     rms_norm_kernel<<<n, 256, 0, stream>>>(in, gamma, out, size, eps);
     return hipGetLastError();
 }
@@ -287,7 +369,39 @@ hipError_t launch_attn_temperature(const float* in, float* out, uint32_t n, uint
 
 hipError_t launch_elementwise(const float* a, const float* b, float* out, uint64_t count, uint32_t op, float scalar,
                               uint32_t period, hipStream_t stream) {
-    elementwise_kernel<<<grid_for(count), 256, 0, stream>>>(a, b, out, count, op, scalar, period);
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool by4 = count % 4 == 0 && aligned(a) && aligned(out) && (!elementwise_reads_b(op) || aligned(b)) &&
+                     (op != elementwise_add_bias || period % 4 == 0);
+    const auto go = [&]<uint32_t OP>() {
+        if (by4) {
+            elementwise_kernel<OP, 4><<<grid_for(count / 4), 256, 0, stream>>>(a, b, out, count, scalar, period);
+        } else {
+            elementwise_kernel<OP, 1><<<grid_for(count), 256, 0, stream>>>(a, b, out, count, scalar, period);
+        }
+    };
+    switch (op) {
+    case elementwise_add:
+        go.template operator()<elementwise_add>();
+        break;
+    case elementwise_mul:
+        go.template operator()<elementwise_mul>();
+        break;
+    case elementwise_silu_mul:
+        go.template operator()<elementwise_silu_mul>();
+        break;
+    case elementwise_gelu:
+        go.template operator()<elementwise_gelu>();
+        break;
+    case elementwise_silu:
+        go.template operator()<elementwise_silu>();
+        break;
+    case elementwise_add_bias:
+        go.template operator()<elementwise_add_bias>();
+        break;
+    default:
+        go.template operator()<elementwise_scale>();
+        break;
+    }
     return hipGetLastError();
 }
 
