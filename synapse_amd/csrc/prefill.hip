@@ -438,7 +438,10 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void prefill_kernel(const f
 // same number of steps, so the block-wide barriers pair up. The two partial
 // (max, sum, O) of the later tile's queries meet in LDS at the end, in a
 // fixed order. The tail of the last V^T chunk past kv_end is zeroed by the
-// lane that copied it, right after its copy lands.
+// lane that copied it, right after its copy lands. 2048 queries of 32 heads on
+// 8, hd 128: 56.2 us (59.5-61.4 with two barriers a tile and the row sums
+// taken across the lane halves on every tile), 612 TFLOP/s; what bounds it is
+// the LDS reads (a wave reads a whole tile for 32 queries) beside the softmax.
 template <int HD, bool QF16>
 __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a) {
     constexpr int NS = HD / 16;
@@ -595,11 +598,11 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
         l_run = 0.0f;
     };
     // The normalised rows of the current query tile, to out.
-    const auto store = [&]() __attribute__((always_inline)) {
+    const auto store = [&](float l) __attribute__((always_inline)) {
         if (my_q >= a.n) {
             return;
         }
-        const float inv = 1.0f / l_run;
+        const float inv = 1.0f / l;
         float* out = a.out + static_cast<std::size_t>(my_q) * a.q_row + h * hd;
         // The dims' bounds compared here, where they are used: hoisted out of
         // the item loop, their lane masks took 32 scalar registers for the
@@ -707,8 +710,7 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
                 psum = add_pair(h2{pv[s2][i], pv[s2][i + 1]}, psum);
             }
         }
-        psum = sum32(psum);
-        l_run = whole ? 1.0f : l_run + psum;
+        l_run = whole ? 0.5f : l_run + psum;  // this lane half's share (whole: 1 together)
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             const char* vrow = sv + ((32 * n + qi) * VROWC + H) * 16;
@@ -716,18 +718,6 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
             for (int s2 = 0; s2 < 4; ++s2) {
                 o[n] = mfma32(*reinterpret_cast<const h8*>(vrow + 32 * s2), pv[s2], o[n]);
             }
-        }
-    };
-
-    // This wave's copies per item: TT / 4 or one more.
-    const uint32_t per_tile = (TT - wg + 3) / 4;
-    const auto wait_item = [&](bool next_issued) __attribute__((always_inline)) {
-        if (!next_issued) {
-            __builtin_amdgcn_s_waitcnt(pf_vmcnt(0));
-        } else if (per_tile == (TT + 3) / 4) {
-            __builtin_amdgcn_s_waitcnt(pf_vmcnt((TT + 3) / 4));
-        } else {
-            __builtin_amdgcn_s_waitcnt(pf_vmcnt(TT / 4));
         }
     };
 
@@ -740,63 +730,57 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
         }
         const uint32_t qt = item_qt(j);
         if (qt != cur_qt) {
-            store();
+            store(sum32(l_run));
             reset();
             enter(qt);
             cur_qt = qt;
         }
         compute.template operator()<false>(item_kt(j) * pf_bk, sk, sv);
     };
-    // The group's pipeline over its items; both groups take `half` steps
-    // (two barriers each), so every barrier has all 8 waves.
-    // The first query tile's q loads go out after the first two items'
-    // copies, and enter's wait covers all of them.
+    // The group's pipeline over its items; both groups take `half` steps, one
+    // barrier each, so every barrier has all 8 waves: item j has landed in
+    // every wave and item j - 1 is read, so item j + 1's copies go out ahead
+    // of item j's products. (Two barriers an item, with the copies of j + 2
+    // going out after the products of j, gave a copy the same time to land.)
+    // The first query tile's q loads go out after the first item's copies, and
+    // enter's wait covers both.
     const auto pipeline = [&](char* k0, char* v0, char* k1, char* v1) __attribute__((always_inline)) {
+        const auto landed = [&](uint32_t j, char* sv) __attribute__((always_inline)) {
+            __builtin_amdgcn_s_waitcnt(pf_vmcnt(0));
+            if (j < cnt) {
+                tail(j, sv);
+            }
+            pf_barrier();
+        };
         if (cnt > 0) {
             issue(0, k0, v0);
         }
+        enter(cur_qt);
+        landed(0, v0);
         if (cnt > 1) {
             issue(1, k1, v1);
         }
-        enter(cur_qt);
-        if (cnt > 0) {
-            tail(0, v0);
-        }
-        pf_barrier();
         // Item 0 apart, the only one that can hold whole-softmax queries, so
-        // the loop's items keep the plain form's registers. The loop is the
-        // same sequence rotated: each item, then its two barriers.
+        // the loop's items keep the plain form's registers.
         if (cnt > 0) {
             compute.template operator()<true>(item_kt(0) * pf_bk, k0, v0);
         }
-        for (uint32_t j = 0; j < half; j += 2) {
-            pf_barrier();
-            if (j + 2 < cnt) {
-                issue(j + 2, k0, v0);
-            }
-            wait_item(j + 2 < cnt);
+        for (uint32_t j = 1; j < half; j += 2) {
+            landed(j, v1);
             if (j + 1 < cnt) {
-                tail(j + 1, v1);
+                issue(j + 1, k0, v0);
             }
-            pf_barrier();
+            run(j, k1, v1);
             if (j + 1 >= half) {
                 break;
             }
-            run(j + 1, k1, v1);
-            pf_barrier();
-            if (j + 3 < cnt) {
-                issue(j + 3, k1, v1);
-            }
-            wait_item(j + 3 < cnt);
+            landed(j + 1, v0);
             if (j + 2 < cnt) {
-                tail(j + 2, v0);
+                issue(j + 2, k1, v1);
             }
-            pf_barrier();
-            if (j + 2 >= half) {
-                break;
-            }
-            run(j + 2, k0, v0);
+            run(j + 1, k0, v0);
         }
+        pf_barrier();  // the merge below reuses the stages
     };
     reset();
     if (grp == 0) {
@@ -807,7 +791,7 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
     // Group 0 may have ended on the earlier tile (it took none of the later
     // tile's keys): its rows go out and its partial of the later tile is empty.
     if (grp == 0 && cur_qt != tB) {
-        store();
+        store(sum32(l_run));
         reset();
         enter(tB);
     }
@@ -829,6 +813,7 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
         }
         return reinterpret_cast<float*>(lv01) + (f - 2 * TK - TV) * 256 + lane;
     };
+    l_run = sum32(l_run);
     if (grp == 0) {
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
@@ -854,7 +839,7 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
                 o[n][i] = *slot(16 * n + i) * a0 + o[n][i] * a1;
             }
         }
-        store();
+        store(l_run);
     }
 }
 
