@@ -288,8 +288,13 @@ hipError_t launch_hd(const flash_args& a, hipStream_t stream) {
 }  // namespace
 
 bool self_f32_mfma_fits(const flash_args& a) {
-    return a.hd % 4 == 0 && uint64_t{a.n} * a.row * 4 < (uint64_t{1} << 31) &&
-           (uint64_t{a.n} + sf_q - 1) / sf_q * a.n_heads * a.batch < (uint64_t{1} << 31);
+    // Rows are read and written 16 bytes at a time (heads of whole 8-dim
+    // chunks are aligned by the interface, those of 4, 12, ... dims need not
+    // be); a launch takes fewer than 2^32 threads in one dimension.
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    return a.hd % 4 == 0 && aligned(a.q) && aligned(a.k_rows) && aligned(a.v_rows) && aligned(a.out) &&
+           uint64_t{a.n} * a.row * 4 < (uint64_t{1} << 31) &&
+           (uint64_t{a.n} + sf_q - 1) / sf_q * a.n_heads * a.batch < (uint64_t{1} << 24);
 }
 
 hipError_t launch_self_f32_mfma(const flash_args& a, hipStream_t stream) {

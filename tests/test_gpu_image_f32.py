@@ -4,11 +4,13 @@ kernel (flash_f32.hip) at the edges of its tiles, and the row-per-wave kernel
 oracle."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
 import binding as orc
-from gpu_util import SYN_F32, Arena, self_attention
+from gpu_util import SYN_F32, Arena, SelfDesc, check, lib, self_attention
 from synapse_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +66,37 @@ def test_image_f32_extreme_scores(arena):
     # which its exponential shows as a relative error.
     top = np.abs((q[rows] @ k.T) * 0.125).max()
     assert np.abs(got[rows] - want[rows]).max() <= max(BOUND, top * 2.0 ** -24 * 8) * np.abs(want[rows]).max()
+
+
+@pytest.mark.parametrize("at", range(4))
+def test_image_f32_offsets(arena, at):
+    """Rows of 12-dim heads on 4-byte offsets, as the interface takes them."""
+    n, heads, hd = 40, 2, 12
+    g = wl.rng(at)
+    rows = [wl.normal(g, (n, heads * hd)) for _ in range(3)]
+    mark = arena.top
+    offs = [arena.alloc(n * heads * hd * 4 + 256) for _ in range(4)]
+    offs[at] += 4
+    for off, x in zip(offs, rows):
+        arena.upload(off, x)
+    d = SelfDesc(q_offset=offs[0], k_offset=offs[1], v_offset=offs[2], out_offset=offs[3], n=n, batch=1, n_heads=heads,
+                 head_dim=hd, scale=0.25, in_dtype=SYN_F32)
+    check(lib().syn_hip_self_attention(arena.handle, ctypes.byref(d)))
+    got = arena.download(offs[3], (n, heads * hd), np.float32)
+    want = orc.self_attention(*rows, heads, 0.25, threads=8)
+    assert np.abs(got - want).max() <= BOUND * np.abs(want).max()
+    arena.top = mark
+
+
+def test_image_f32_many_small_images():
+    """More 16-row tiles than one launch dimension takes in blocks of 256
+    threads: one key each, so the output is v."""
+    batch, heads, hd = 65535, 257, 4
+    assert batch * heads >= 2 ** 24
+    x = np.arange(batch * heads * hd, dtype=np.float32).reshape(batch, heads * hd) % 8191
+    with Arena(3 * x.nbytes) as a:
+        off, out = a.put(x), a.alloc(x.nbytes)
+        d = SelfDesc(q_offset=off, k_offset=off, v_offset=off, out_offset=out, n=1, batch=batch, n_heads=heads,
+                     head_dim=hd, scale=2.0 ** -30, in_dtype=SYN_F32)
+        check(lib().syn_hip_self_attention(a.handle, ctypes.byref(d)))
+        assert np.array_equal(a.download(out, x.shape, np.float32), x)
