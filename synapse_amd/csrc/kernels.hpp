@@ -323,7 +323,7 @@ uint64_t qtype_act_bytes(uint32_t t, uint32_t n, uint32_t cols);    // quantized
 constexpr uint32_t matmul_q_max_lds = 160 * 1024;
 // Whether the quantized product of n activation rows runs as a GEMM on the
 // int8 matrix cores instead of passes of the GEMV.
-bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t cols);
+bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t rows, uint32_t cols);
 uint32_t matmul_q_rows_per_pass(uint32_t n, uint32_t cols);
 // The same product for many activation rows on the int8 matrix cores
 // (quantizes x into act first).

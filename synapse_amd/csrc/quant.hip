@@ -486,7 +486,7 @@ gemv_occupancy* gemv_occupancy_of(int dev, const void* kernel, uint32_t lds) {
 
 hipError_t launch_matmul_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
                            uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream) {
-    if (gemm_q_takes(t, w, act, n, cols)) {
+    if (gemm_q_takes(t, w, act, n, rows, cols)) {
         return launch_gemm_q(t, w, x, act, bias, out, n, rows, cols, stream);
     }
     const uint32_t nr = matmul_q_rows_per_pass(n, cols);

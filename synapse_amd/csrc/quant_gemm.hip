@@ -1645,6 +1645,10 @@ bool staged_ok(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t cols) 
            (cols % 64 == 0 && (reinterpret_cast<uintptr_t>(w) & 3) == 0 && (reinterpret_cast<uintptr_t>(act) & 3) == 0);
 }
 
+// gemm_r16_kernel launches 32 threads per weight row, and a launch takes fewer
+// than 2^32 of them (the GEMV's grid is a resident one).
+constexpr uint32_t r16_max_rows = (1u << 27) - 16;
+
 // Calls go.operator()<T>() for the weight type.
 template <class F>
 void for_qtype(uint32_t t, const F& go) {
@@ -1675,8 +1679,8 @@ void for_qtype(uint32_t t, const F& go) {
 // 2 rows 16.8 / 12.8, 14.3 / 13.6, 7.9 / 7.9; Q6_K 19.3 / 16.7, 16.5 / 17.8,
 // 9.3 / 9.0; Q8_0 22.7 / 18.9, 16.9 / 19.5, 11.0 / 9.3: even at two rows; at
 // four Q4_K 23.7 / 12.8, 22.6 / 14.3, 12.2 / 8.3.
-bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t cols) {
-    return n >= (staged_ok(t, w, act, cols) ? 3u : 32u);
+bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t rows, uint32_t cols) {
+    return n >= (staged_ok(t, w, act, cols) && rows < r16_max_rows ? 3u : 32u);
 }
 
 hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
@@ -1694,7 +1698,7 @@ hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* 
     // at 24 rows, GEMV passes against these tiles: Q6_K 4096 x 14336 147 /
     // 22, 14336 x 4096 112 / 29; Q4_K 112 / 18, 110 / 23; Q8_0 133 / 27, 90 /
     // 33; 1024 x 4096 30 / 9 (Q4_K).
-    if (staged && n <= 32) {
+    if (staged && n <= 32 && rows < r16_max_rows) {
         const uint32_t tiles = (rows + 15) / 16;
         for_qtype(t, [&]<uint32_t T>() {
             if (n <= 16) {

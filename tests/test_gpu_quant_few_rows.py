@@ -3,11 +3,13 @@ matrix-core kernels whose waves split the columns (gemm_r16_kernel up to 32
 rows, gemm_ks_kernel above), at the edges of their tiles, units and rules."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
 import quant_host as qh
-from gpu_util import Arena
+from gpu_util import Arena, capi, check, lib
 from synapse_amd.gguf import BLOCK, Q4_0, Q4_K, Q5_0, Q6_K, Q8_0
 from test_gpu_quant import matmul_q, random_blocks
 
@@ -95,3 +97,28 @@ def test_extreme_weights(arena, n):
         xa = np.stack([qh.dequantize_act(a, qh.act_type(t)) for a in act]).astype(np.float64)
         err = np.abs(out - xa @ w.T)
         assert np.all(err <= 1e-5 * np.maximum(np.abs(xa) @ np.abs(w).T, 1.0))
+
+
+def test_more_rows_than_one_launch():
+    """16-row tiles take 32 threads per weight row, which 2^27 rows are too
+    many for: the GEMV does them."""
+    t, n, rows, cols, last = Q4_0, 3, 1 << 27, 64, 40
+    rng = np.random.default_rng(27)
+    raw = random_blocks(t, last, cols, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    wbytes = rows * (cols // 32) * BLOCK[t][1]
+    with Arena(wbytes + n * rows * 4 + (1 << 20)) as a:
+        wo = a.alloc(wbytes)
+        a.fill(wo, 0, wbytes)
+        a.upload(wo + wbytes - raw.nbytes, raw)
+        xo, act = a.put(x), a.alloc(4096)
+        oo = a.alloc(n * rows * 4)
+        d = capi.MatmulQDesc(w_offset=wo, x_offset=xo, act_offset=act, bias_offset=capi.NO_OFFSET, out_offset=oo,
+                             w_type=t, n=n, rows=rows, cols=cols)
+        check(lib().syn_hip_matmul_q(a.handle, ctypes.byref(d)))
+        w = qh.dequantize(raw, t).reshape(last, cols).astype(np.float64)
+        for r in range(n):
+            xa = qh.dequantize_act(qh.quantize_act(x[r], t), qh.act_type(t)).astype(np.float64)
+            got = a.download(oo + 4 * ((r + 1) * rows - 2 * last), (2 * last,), np.float32)
+            assert not got[:last].any()
+            assert np.all(np.abs(got[last:] - w @ xa) <= 1e-5 * np.maximum(np.abs(w) @ np.abs(xa), 1.0))
