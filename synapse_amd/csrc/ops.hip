@@ -332,7 +332,8 @@ hipError_t launch_rms_norm(const float* in, const float* gamma, float* out, uint
         // As few threads as hold the row: one row of 4096 takes 2.2 us with
         // 256 (2.5 with 1024, 5.5 in the row-loop form), 2048 rows 10.7 (14.3,
         // 16.9); replayed from a graph.
-        const bool held = size <= 1024 * 16;
+        // (A launch takes fewer than 2^32 threads.)
+        const bool held = size <= 256 * 16 || (size <= 1024 * 16 && n < (1u << 22));
         if (size <= 256 * 4) {
             rms_norm_vec_kernel<256, 1><<<n, 256, 0, stream>>>(in, gamma, out, size, eps);
         } else if (size <= 256 * 16) {
