@@ -1225,20 +1225,27 @@ __global__ __launch_bounds__(256) void gemm_ks_kernel(const uint8_t* w, const ui
     lds_barrier();
 
     // ---- the four waves' sums, in order; wave v writes rows 8 v .. 8 v + 7 -----------------
+    // (Added in double, rounded once: with a unit or two per wave float sums
+    // here would be the larger part of the error.)
     f4* part = reinterpret_cast<f4*>(lds);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         part[(wv * 4 + q) * 64 + ln] = f4{acc[0][4 * q], acc[0][4 * q + 1], acc[0][4 * q + 2], acc[0][4 * q + 3]};
     }
     lds_barrier();
-    f4 sum = part[wv * 64 + ln];
+    double merged[4] = {};
 #pragma unroll
-    for (int v = 1; v < 4; ++v) {
+    for (int v = 0; v < 4; ++v) {
         const f4 p = part[(v * 4 + wv) * 64 + ln];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            sum[i] += p[i];
+            merged[i] += static_cast<double>(p[i]);
         }
+    }
+    f4 sum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sum[i] = static_cast<float>(merged[i]);
     }
     const uint32_t o = o0 + li;
     if (o < rows) {
@@ -1526,6 +1533,10 @@ __global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const u
         } else {
             // Blocks of 32: v_mfma_i32_16x16x32_i8, lane group G columns 8 G
             // .. 8 G + 7. The activation scales go to LDS as f32 [block][row].
+            // A unit's blocks sum from zero, so that no chain is longer than 8
+            // blocks or the wave's units (7.2e-8 against 64 bits at 8192 columns;
+            // in one chain 1.17e-7, where the GEMV has 8.2e-8).
+            f4 usum[AT] = {};
             const uint32_t nblk = min(8u, cols / 32 - 8 * U);
             float* da = reinterpret_cast<float*>(S + ST::d);
 #pragma unroll
@@ -1577,7 +1588,7 @@ __global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const u
                     const f4 d4 = *reinterpret_cast<const f4*>(da + AR * b + 16 * t + 4 * G);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        acc[t][r] += static_cast<float>(cm[r]) * (dw * d4[r]);
+                        usum[t][r] += static_cast<float>(cm[r]) * (dw * d4[r]);
                     }
                 }
             };
@@ -1594,6 +1605,10 @@ __global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const u
             part.template operator()<5>();
             part.template operator()<6>();
             part.template operator()<7>();
+#pragma unroll
+            for (int t = 0; t < AT; ++t) {
+                acc[t] += usum[t];
+            }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (U + NW < units) {
                 issue(U + NW);
@@ -1601,7 +1616,7 @@ __global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const u
         }
     }
 
-    // ---- the eight waves' sums, in order: wave v adds tile v's ------------------------------
+    // ---- the eight waves' sums, in order and in double: wave v adds tile v's ----------------
     lds_barrier();
     f4* part = reinterpret_cast<f4*>(lds);
 #pragma unroll
@@ -1612,14 +1627,19 @@ __global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const u
     if (wv >= AT) {
         return;
     }
-    f4 sum = part[wv * 64 + ln];
+    double merged[4] = {};
 #pragma unroll
-    for (uint32_t v = 1; v < NW; ++v) {
+    for (uint32_t v = 0; v < NW; ++v) {
         const f4 p = part[(v * AT + wv) * 64 + ln];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            sum[r] += p[r];
+            merged[r] += static_cast<double>(p[r]);
         }
+    }
+    f4 sum;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        sum[r] = static_cast<float>(merged[r]);
     }
     const uint32_t o = o0 + c;
     if (o < rows) {
@@ -1719,7 +1739,11 @@ hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* 
     // tiles) 244 / 212, 14336 x 4096 at 128 (1792) 78 / 65, at 256 93 / 114.
     const uint32_t act_tiles = (n + 31) / 32;
     const uint64_t tiles = uint64_t{(rows + 31) / 32} * act_tiles;
-    if (staged && tiles <= (kq ? 1024u : 2048u)) {
+    // Up to three 256-blocks a row give a wave one block at most: the larger
+    // tiles' one running sum is then as exact (768 columns, error against 64
+    // bits 5.1e-8 in those, 5.2e-8 in these; from four blocks on these have
+    // the smaller one).
+    if (staged && tiles <= (kq ? 1024u : 2048u) && (!kq || cols >= 1024)) {
         for_qtype(t, [&]<uint32_t T>() {
             gemm_ks_kernel<T><<<static_cast<uint32_t>(tiles), 256, 0, stream>>>(w, act, bias, out, n, rows, cols,
                                                                                 act_tiles);

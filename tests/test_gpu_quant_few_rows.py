@@ -47,7 +47,8 @@ def test_few_rows(arena, t, n, rows, cols):
 
 
 # The last count of 32 x 32 tiles that gemm_ks_kernel takes, and one row more.
-@pytest.mark.parametrize("t,rows,cols", [(Q4_K, 16384, 256), (Q4_K, 16385, 256), (Q6_K, 16384, 256), (Q6_K, 16385, 256),
+@pytest.mark.parametrize("t,rows,cols", [(Q4_K, 16384, 1024), (Q4_K, 16385, 1024), (Q6_K, 16384, 1024),
+                                         (Q6_K, 16385, 1024), (Q4_K, 16, 768),
                                          (Q8_0, 32768, 64), (Q8_0, 32769, 64)])
 def test_tile_count_rule(arena, t, rows, cols):
     _check(arena, t, 33, rows, cols)
