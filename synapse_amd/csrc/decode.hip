@@ -113,27 +113,6 @@ struct decode_traits<decode_batch_args> {
     }
 };
 
-// LDS of the split kernel: the group's q as given (f32 size, the larger),
-// the new K and V row of one head (likewise), per-wave (max, sum), the
-// waves' unscaled outputs (head rows padded by 4 floats), then a fused
-// step's RoPE table (hd/2 cos, hd/2 sin), frequency factors (a 1 KB copy)
-// and the pairs' angles.
-inline __host__ __device__ uint32_t q_lds_bytes(uint32_t group, uint32_t hd) {
-    return (group * hd * 4 + 15) / 16 * 16;
-}
-inline __host__ __device__ uint32_t new_lds_bytes(uint32_t hd) {
-    return (2 * hd * 4 + 15) / 16 * 16;
-}
-// (max, sum) slots: 4 waves and the new row, 16 heads each; then the 4
-// waves' parts of the new row's scores, 16 heads each.
-constexpr uint32_t decode_ml_floats = 5 * 16 * 2 + 4 * 16;
-inline __host__ __device__ uint32_t rope_lds_offset(uint32_t group, uint32_t hd) {
-    return q_lds_bytes(group, hd) + new_lds_bytes(hd) + (decode_ml_floats + 4 * group * (hd + 4)) * 4;
-}
-inline std::size_t decode_lds_bytes(uint32_t group, uint32_t hd) {
-    return rope_lds_offset(group, hd) + std::size_t{hd} * sizeof(float) + 1024 + rope_max_pairs * sizeof(float);
-}
-
 // s_waitcnt immediate that waits until at most n vector memory operations
 // are outstanding (gfx9 encoding: vmcnt split over bits 3:0 and 15:14;
 // expcnt and lgkmcnt left at their no-wait maxima).
@@ -224,7 +203,8 @@ __global__ __launch_bounds__(256, SHORT && HDP <= 128 ? 2 : 1) void decode_kerne
     const uint32_t q_bytes = group * hd * (QF16 ? 2 : 4);
     const char* q_src = static_cast<const char*>(s.q) + static_cast<std::size_t>(h0) * hd * (QF16 ? 2 : 4);
     for (uint32_t c0 = 1024 * w; c0 < q_bytes; c0 += 4096) {
-        // q_bytes is a multiple of 16; a lane past its end re-reads chunk 0.
+        // q_bytes is a multiple of 16; a lane past its end re-reads chunk 0
+        // into the rest of q's area (decode_lds.hpp).
         const uint32_t off = c0 + 16 * ln < q_bytes ? c0 + 16 * ln : 0;
         load16_lds(q_src + off, lds_bytes + c0);
     }

@@ -3,6 +3,7 @@
 // C ABI (capi.hip) validates every shape and offset before calling one.
 #pragma once
 
+#include "decode_lds.hpp"
 #include "device.hpp"
 #include "rope_math.hpp"
 
@@ -102,7 +103,6 @@ struct decode_rope_args {
 hipError_t launch_decode(const decode_rope_args& a, uint32_t q_dtype, hipStream_t stream);
 
 
-constexpr uint32_t rope_max_pairs = 128;  // head_dim <= 256, as attention's
 
 // The angles of RoPE pairs 0 .. n_pairs-1 at position pos, as rope() builds
 // them (S/kernels/attention.hpp:101-127): pos times theta_scale p times over

@@ -81,6 +81,12 @@ def test_rope_sin_cos_correctly_rounded():
     _run("test_rope_math")
 
 
+def test_decode_copies_stay_in_their_lds_areas():
+    """The decode kernel's waves copy q and the new row into LDS at once: no
+    copy's tail reaches bytes that another wave's copy or table fills."""
+    _run("test_decode_lds")
+
+
 def test_session_run_allocates_nothing():
     """session::run under a counting operator new, against a C ABI that
     launches nothing (tests/sdk/graph_no_alloc.cpp:199-263 restated)."""
