@@ -95,8 +95,8 @@ CPP_TESTS = {
     "test_session": ("tests/cpp/test_session.cpp", True),
     "test_model_session": ("tests/cpp/test_model_session.cpp", False),
 }
-# Host builds of device-side math and layouts (no library, no HIP).
-CPP_MATH_TESTS = {"test_rope_math": "tests/cpp/test_rope_math.cpp", "test_decode_lds": "tests/cpp/test_decode_lds.cpp"}
+# Host builds of device-side math, layouts and launch rules (no library, no HIP).
+CPP_MATH_TESTS = {name: f"tests/cpp/{name}.cpp" for name in ("test_rope_math", "test_decode_lds", "test_matmul_f32_plan")}
 # Host tests linked against tests/cpp/stub_abi.cpp (a C ABI that launches
 # nothing) instead of the library: they run on the CPU.
 CPP_STUB_TESTS = {"test_no_alloc": "tests/cpp/test_no_alloc.cpp"}

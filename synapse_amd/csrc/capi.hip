@@ -1034,8 +1034,10 @@ int syn_hip_matmul(syn_arena* a, const syn_matmul_desc* d) {
     if (d->rows == 0 || d->cols == 0 || d->n > 65535) {
         return fail(SYN_HIP_EINVAL, "matmul: %u x %u weights, %u rows", d->rows, d->cols, d->n);
     }
+    // The same longest row as syn_hip_matmul_q's, whose GEMV holds it in LDS
+    // (far inside the F32 kernels' own 32-bit limits, matmul_f32_plan.hpp).
     if (syn::matmul_q_rows_per_pass(1, d->cols) == 0) {
-        return fail(SYN_HIP_EUNSUPPORTED, "matmul_q: %u columns exceed the activation LDS", d->cols);
+        return fail(SYN_HIP_EUNSUPPORTED, "matmul: %u columns, more than the interface's longest row", d->cols);
     }
     if (d->n == 0) {
         return SYN_HIP_OK;

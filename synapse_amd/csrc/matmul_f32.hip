@@ -2,7 +2,7 @@
 // x[r][c] (+ bias[o]) (session::execute(op_matmul), S/graph/session.hpp:
 // 287-302; op_add_bias, :306-312), f32 operands, products and sums.
 //
-// Two kernels, by the number of activation rows (on_matrix_cores):
+// Two kernels, by the number of activation rows (matmul_f32_plan.hpp):
 // - gemv_f32_kernel, few rows (a decode step): bound by reading w once. One
 //   wave per weight row, 16 loads in flight; up to four activation rows share
 //   a pass over w.
@@ -10,6 +10,7 @@
 //   f32 matrix cores. Tiles through LDS, v_mfma_f32_32x32x2_f32.
 
 #include "kernels.hpp"
+#include "matmul_f32_plan.hpp"
 
 namespace syn {
 
@@ -246,44 +247,29 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* w, const flo
     }
 }
 
-// The matrix-core kernel's time for few rows is its stages' latency (6 ns per
-// column), the other's grows with n rows cols (0.15 us per million): they
-// meet at n rows = 40000. us per call, one wave per weight row against
-// tiles: 768 x 3072 weights 12.3 / 19.9 at 32 rows, 22.7 / 22.8 at 64; 3072 x
-// 768 5.9 / 6.7 at 8 and 9.7 / 8.0 at 16; 1152 x 588 7.3 / 7.7 at 32, 12.7 /
-// 8.1 at 64. Fewer than 8 rows would leave three quarters of a tile empty.
-bool on_matrix_cores(uint32_t n, uint32_t rows, uint32_t cols) {
-    // (The tiled kernel copies whole 16-byte chunks of a row.)
-    return n >= 8 && uint64_t{n} * rows >= 40000 && cols % 4 == 0;
-}
-
 }  // namespace
 
 hipError_t launch_matmul(const float* w, const float* x, const float* bias, float* out, uint32_t n, uint32_t rows,
                          uint32_t cols, hipStream_t stream) {
-    const auto tiles = [&](uint32_t bm, uint32_t bn) { return ((n + bm - 1) / bm) * uint64_t{(rows + bn - 1) / bn}; };
-    if (on_matrix_cores(n, rows, cols) && tiles(32, 32) < (uint64_t{1} << 31)) {
-        const auto go = [&](auto kernel, uint32_t bm, uint32_t bn) {
-            kernel<<<static_cast<uint32_t>(tiles(bm, bn)), 256, 0, stream>>>(w, x, bias, out, n, rows, cols,
-                                                                             (n + bm - 1) / bm);
+    const matmul_f32_plan p = plan_matmul_f32(n, rows, cols);
+    if (p.blocks_x == 0) {
+        return hipErrorInvalidConfiguration;
+    }
+    if (p.bm != 0) {
+        const auto go = [&](auto kernel) {
+            kernel<<<p.blocks_x, 256, 0, stream>>>(w, x, bias, out, n, rows, cols, (n + p.bm - 1) / p.bm);
         };
-        // The largest tile whose count still fills the 256 CUs (the waves
-        // then split the columns). us per call for 64 x 64, 32 x 64 and
-        // 32 x 32 tiles (with one running sum): 1024 rows of 3072 x 768 45.4,
-        // 50.4, 60.4 (768 tiles of 64 x 64); 512 rows 31.8, 28.3, 33.7 (384
-        // and 768); 729 rows of 768 x 3072 61.1, 57.9, 53.1 (144, 276, 552);
-        // 257 rows of 768 x 768 18.0, 11.6, 8.1.
-        if (tiles(64, 64) >= 512) {
-            go(gemm_f32_kernel<2, 2, 1>, 64, 64);
-        } else if (tiles(32, 64) >= 384) {
-            go(gemm_f32_kernel<1, 2, 2>, 32, 64);
+        if (p.bm == 64) {
+            go(gemm_f32_kernel<2, 2, 1>);
+        } else if (p.bn == 64) {
+            go(gemm_f32_kernel<1, 2, 2>);
         } else {
-            go(gemm_f32_kernel<1, 1, 4>, 32, 32);
+            go(gemm_f32_kernel<1, 1, 4>);
         }
         return hipGetLastError();
     }
     const uint32_t nr = n >= 4 ? 4 : (n >= 2 ? 2 : 1);
-    const dim3 grid((rows + 3) / 4, (n + nr - 1) / nr);
+    const dim3 grid(p.blocks_x, p.blocks_y);
     if (nr == 4) {
         gemv_f32_kernel<4><<<grid, 256, 0, stream>>>(w, x, bias, out, n, rows, cols);
     } else if (nr == 2) {

@@ -23,13 +23,14 @@ def arena():
 # Few rows (one wave per weight row; any column count, row starts on any
 # dword), the last such and the first on the matrix cores (8 rows and
 # n rows >= 40000), then 32 x 32, 32 x 64 and 64 x 64 tiles: whole, one row or
-# one column chunk over, one stage, a partial last stage, columns that are no
+# one column chunk over, one stage, a partial last stage, the longest row the
+# interface takes, columns that are no
 # whole chunks; with and without bias.
 @pytest.mark.parametrize("n,rows,cols", [(1, 1, 1), (1, 5, 3), (1, 70, 1025), (1, 33, 2048), (2, 9, 300), (3, 9, 257),
                                          (4, 40, 768), (7, 6000, 36), (15, 34, 5632), (8, 4999, 64), (8, 5000, 64),
                                          (40, 1000, 4), (40, 1000, 130), (52, 770, 132), (64, 768, 3072),
                                          (257, 768, 768), (100, 9000, 36), (385, 2050, 260), (1000, 1030, 128),
-                                         (1024, 2048, 100), (1025, 2049, 64)])
+                                         (1024, 2048, 100), (1025, 2049, 64), (1, 3, 119167), (64, 640, 20000)])
 def test_matmul_f32(arena, n, rows, cols):
     g = wl.rng(7 * n + rows + cols)
     w, x, b = wl.normal(g, (rows, cols)), wl.normal(g, (n, cols)), wl.normal(g, (rows,))

@@ -87,6 +87,12 @@ def test_decode_copies_stay_in_their_lds_areas():
     _run("test_decode_lds")
 
 
+def test_f32_product_launches_stay_in_range():
+    """The F32 product's choice of kernel at its edges: launches below 2^32
+    threads that cover the product, offsets within 32 bits."""
+    _run("test_matmul_f32_plan")
+
+
 def test_session_run_allocates_nothing():
     """session::run under a counting operator new, against a C ABI that
     launches nothing (tests/sdk/graph_no_alloc.cpp:199-263 restated)."""
