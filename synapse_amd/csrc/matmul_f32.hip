@@ -39,10 +39,13 @@ __device__ __forceinline__ float mf_wave_sum(float v) {
 // One row of 16000 x 2048 21.5 us (6.1 TB/s), 5632 x 2048 8.8, 2048 x 5632
 // 8.9 us; with one load in flight per lane 39.4, 17.7 and 41.0.
 // Row resources end at the row, so columns past it add zeros.
-template <int NR>
+// U loads are in flight per lane: as many as the row has for a lane, at most
+// 16 (a load past the row costs its issue all the same: 20000 x 16 with 3
+// rows 6.2 us a call, 15.5 with 16 loads whatever the row has; one load at a
+// time, one row per pass: 7.2). The order of the sums is the same.
+template <int NR, int U>
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* w, const float* x, const float* bias, float* out,
                                                        uint32_t n, uint32_t rows, uint32_t cols) {
-    constexpr int U = 16;  // weight loads in flight per lane
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t ln = threadIdx.x & 63;
     const uint32_t o = blockIdx.x * 4 + wv;
@@ -270,12 +273,24 @@ hipError_t launch_matmul(const float* w, const float* x, const float* bias, floa
     }
     const uint32_t nr = n >= 4 ? 4 : (n >= 2 ? 2 : 1);
     const dim3 grid(p.blocks_x, p.blocks_y);
+    const auto gemv = [&]<int NR>() {
+        const auto go = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>(w, x, bias, out, n, rows, cols); };
+        if (cols <= 64) {
+            go(gemv_f32_kernel<NR, 1>);
+        } else if (cols <= 256) {
+            go(gemv_f32_kernel<NR, 4>);
+        } else if (cols <= 512) {
+            go(gemv_f32_kernel<NR, 8>);
+        } else {
+            go(gemv_f32_kernel<NR, 16>);
+        }
+    };
     if (nr == 4) {
-        gemv_f32_kernel<4><<<grid, 256, 0, stream>>>(w, x, bias, out, n, rows, cols);
+        gemv.template operator()<4>();
     } else if (nr == 2) {
-        gemv_f32_kernel<2><<<grid, 256, 0, stream>>>(w, x, bias, out, n, rows, cols);
+        gemv.template operator()<2>();
     } else {
-        gemv_f32_kernel<1><<<grid, 256, 0, stream>>>(w, x, bias, out, n, rows, cols);
+        gemv.template operator()<1>();
     }
     return hipGetLastError();
 }

@@ -26,7 +26,8 @@ def arena():
 # one column chunk over, one stage, a partial last stage, the longest row the
 # interface takes, columns that are no
 # whole chunks; with and without bias.
-@pytest.mark.parametrize("n,rows,cols", [(1, 1, 1), (1, 5, 3), (1, 70, 1025), (1, 33, 2048), (2, 9, 300), (3, 9, 257),
+@pytest.mark.parametrize("n,rows,cols", [(1, 1, 1), (1, 5, 3), (1, 70, 1025), (1, 33, 2048), (2, 9, 64), (7, 70, 65),
+                                         (1, 9, 256), (5, 9, 257), (3, 6, 512), (4, 6, 513), (2, 9, 300), (3, 9, 257),
                                          (4, 40, 768), (7, 6000, 36), (15, 34, 5632), (8, 4999, 64), (8, 5000, 64),
                                          (40, 1000, 4), (40, 1000, 130), (52, 770, 132), (64, 768, 3072),
                                          (257, 768, 768), (100, 9000, 36), (385, 2050, 260), (1000, 1030, 128),
