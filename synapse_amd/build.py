@@ -96,7 +96,8 @@ CPP_TESTS = {
     "test_model_session": ("tests/cpp/test_model_session.cpp", False),
 }
 # Host builds of device-side math, layouts and launch rules (no library, no HIP).
-CPP_MATH_TESTS = {name: f"tests/cpp/{name}.cpp" for name in ("test_rope_math", "test_decode_lds", "test_matmul_f32_plan")}
+CPP_MATH_TESTS = {name: f"tests/cpp/{name}.cpp"
+                  for name in ("test_rope_math", "test_decode_lds", "test_matmul_f32_plan", "test_quant_plan")}
 # Host tests linked against tests/cpp/stub_abi.cpp (a C ABI that launches
 # nothing) instead of the library: they run on the CPU.
 CPP_STUB_TESTS = {"test_no_alloc": "tests/cpp/test_no_alloc.cpp"}

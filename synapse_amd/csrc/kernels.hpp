@@ -5,6 +5,7 @@
 
 #include "decode_lds.hpp"
 #include "device.hpp"
+#include "quant_plan.hpp"
 #include "rope_math.hpp"
 
 #include <cstddef>
@@ -312,8 +313,7 @@ hipError_t launch_attn_temperature(const float* in, float* out, uint32_t n, uint
 hipError_t launch_elementwise(const float* a, const float* b, float* out, uint64_t count, uint32_t op, float scalar,
                               uint32_t period,
                               hipStream_t stream);
-// Quantized weights (quant.hip), ggml type numbers.
-constexpr uint32_t qtype_q4_0 = 2, qtype_q5_0 = 6, qtype_q8_0 = 8, qtype_q4_k = 12, qtype_q6_k = 14;
+// Quantized weights (quant.hip).
 bool qtype_known(uint32_t t);
 uint32_t qtype_block(uint32_t t);                                   // elements per block
 uint64_t qtype_row_bytes(uint32_t t, uint32_t cols);                // bytes of one row of cols
@@ -321,14 +321,13 @@ uint64_t qtype_act_bytes(uint32_t t, uint32_t n, uint32_t cols);    // quantized
 // LDS a quantized matmul may take for its activation rows (an 8-wave
 // workgroup), and the activation rows one pass can carry (0: cols too long).
 constexpr uint32_t matmul_q_max_lds = 160 * 1024;
-// Whether the quantized product of n activation rows runs as a GEMM on the
-// int8 matrix cores instead of passes of the GEMV.
-bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t rows, uint32_t cols);
 uint32_t matmul_q_rows_per_pass(uint32_t n, uint32_t cols);
-// The same product for many activation rows on the int8 matrix cores
-// (quantizes x into act first).
-hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
-                         uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream);
+// The same product on the int8 matrix cores by the named kernel
+// (plan_matmul_q; quantizes x into act first), and whether the operands take
+// the staged kernels' copies.
+bool matmul_q_staged(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t cols);
+hipError_t launch_gemm_q(quant_kernel kernel, uint32_t t, const uint8_t* w, const float* x, uint8_t* act,
+                         const float* bias, float* out, uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream);
 hipError_t launch_matmul_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
                            uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream);
 hipError_t launch_embed_q(uint32_t t, const uint8_t* table, float* out, const embed_tokens& tk, uint32_t n,

@@ -486,23 +486,22 @@ gemv_occupancy* gemv_occupancy_of(int dev, const void* kernel, uint32_t lds) {
 
 hipError_t launch_matmul_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
                            uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream) {
-    if (gemm_q_takes(t, w, act, n, rows, cols)) {
-        return launch_gemm_q(t, w, x, act, bias, out, n, rows, cols, stream);
-    }
     const uint32_t nr = matmul_q_rows_per_pass(n, cols);
     if (nr == 0) {
         return hipErrorInvalidValue;
+    }
+    const uint32_t cus = device_cu_count();  // (0: not known, and only the GEMV needs it)
+    const quant_kernel which =
+        plan_matmul_q(t, matmul_q_staged(t, w, act, cols), n, nr, rows, cols, cus != 0 ? cus : 256);
+    if (which != quant_kernel::gemv) {
+        return launch_gemm_q(which, t, w, x, act, bias, out, n, rows, cols, stream);
     }
     const uint32_t lds = gemv_lds_bytes(nr, cols / 32);
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) {
         return e;
     }
-    if (dev < 0 || dev >= gemv_max_devices) {
-        return hipErrorInvalidDevice;
-    }
-    const uint32_t cus = device_cu_count();
-    if (cus == 0) {
+    if (dev < 0 || dev >= gemv_max_devices || cus == 0) {
         return hipErrorInvalidDevice;
     }
     const auto go = [&]<uint32_t T>() {

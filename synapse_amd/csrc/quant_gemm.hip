@@ -14,7 +14,8 @@
 //   Q6_K               per 256-block: (d yd) (float(sum_k sc_k sumi_k) - 32 sum_k sc_k bsum_k)
 //
 // so each block's integers are ggml's and results differ from its gemv only
-// by float association. The kernels, chosen in launch_gemm_q:
+// by float association. The kernels, chosen by plan_matmul_q
+// (quant_plan.hpp):
 // - gemm_r16_kernel (all formats, up to 32 activation rows) and gemm_ks_kernel
 //   (all formats, few 32 x 32 tiles): the columns split over a block's waves.
 // - gemm_q4k_kernel (Q4_K): a workgroup (4 waves) owns 128 weight rows x 64
@@ -1657,18 +1658,6 @@ __global__ __launch_bounds__(512) void gemm_r16_kernel(const uint8_t* w, const u
 
 namespace {
 
-// The 32-block formats' staged kernels copy row windows of whole blocks: every
-// unit of two blocks starts on a dword when cols is a multiple of 64 (w and
-// act are 4-byte aligned, as the interface keeps them).
-bool staged_ok(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t cols) {
-    return t == qtype_q4_k || t == qtype_q6_k ||
-           (cols % 64 == 0 && (reinterpret_cast<uintptr_t>(w) & 3) == 0 && (reinterpret_cast<uintptr_t>(act) & 3) == 0);
-}
-
-// gemm_r16_kernel launches 32 threads per weight row, and a launch takes fewer
-// than 2^32 of them (the GEMV's grid is a resident one).
-constexpr uint32_t r16_max_rows = (1u << 27) - 16;
-
 // Calls go.operator()<T>() for the weight type.
 template <class F>
 void for_qtype(uint32_t t, const F& go) {
@@ -1693,18 +1682,16 @@ void for_qtype(uint32_t t, const F& go) {
 
 }  // namespace
 
-// The GEMV passes over the weights once per four activation rows and decodes
-// them on the way for each; a matrix-core tile takes 16. us per call (4096 x
-// 14336, 14336 x 4096, 4096 x 4096 weights), GEMV against 16-row tiles: Q4_K
-// 2 rows 16.8 / 12.8, 14.3 / 13.6, 7.9 / 7.9; Q6_K 19.3 / 16.7, 16.5 / 17.8,
-// 9.3 / 9.0; Q8_0 22.7 / 18.9, 16.9 / 19.5, 11.0 / 9.3: even at two rows; at
-// four Q4_K 23.7 / 12.8, 22.6 / 14.3, 12.2 / 8.3.
-bool gemm_q_takes(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t n, uint32_t rows, uint32_t cols) {
-    return n >= (staged_ok(t, w, act, cols) && rows < r16_max_rows ? 3u : 32u);
+// The 32-block formats' staged kernels copy row windows of whole blocks: every
+// unit of two blocks starts on a dword when cols is a multiple of 64 (w and
+// act are 4-byte aligned, as the interface keeps them).
+bool matmul_q_staged(uint32_t t, const uint8_t* w, const uint8_t* act, uint32_t cols) {
+    return t == qtype_q4_k || t == qtype_q6_k ||
+           (cols % 64 == 0 && (reinterpret_cast<uintptr_t>(w) & 3) == 0 && (reinterpret_cast<uintptr_t>(act) & 3) == 0);
 }
 
-hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* act, const float* bias, float* out,
-                         uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream) {
+hipError_t launch_gemm_q(quant_kernel kernel, uint32_t t, const uint8_t* w, const float* x, uint8_t* act,
+                         const float* bias, float* out, uint32_t n, uint32_t rows, uint32_t cols, hipStream_t stream) {
     const bool kq = t == qtype_q4_k || t == qtype_q6_k;
     const uint64_t total = uint64_t{n} * (cols / 32);
     const uint32_t qblocks = static_cast<uint32_t>((total + 255) / 256);
@@ -1713,12 +1700,7 @@ hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* 
     } else {
         quantize_act_kernel<false><<<qblocks, 256, 0, stream>>>(x, act, n, cols);
     }
-    const bool staged = staged_ok(t, w, act, cols);
-    // Up to 32 rows: 16-row weight tiles, the weights read once. us per call
-    // at 24 rows, GEMV passes against these tiles: Q6_K 4096 x 14336 147 /
-    // 22, 14336 x 4096 112 / 29; Q4_K 112 / 18, 110 / 23; Q8_0 133 / 27, 90 /
-    // 33; 1024 x 4096 30 / 9 (Q4_K).
-    if (staged && n <= 32 && rows < r16_max_rows) {
+    if (kernel == quant_kernel::r16) {
         const uint32_t tiles = (rows + 15) / 16;
         for_qtype(t, [&]<uint32_t T>() {
             if (n <= 16) {
@@ -1729,27 +1711,15 @@ hipError_t launch_gemm_q(uint32_t t, const uint8_t* w, const float* x, uint8_t* 
         });
         return hipGetLastError();
     }
-    // While a product is few tiles of 32 x 32, those with the columns split
-    // over the waves; beyond, the larger tiles decode a weight for more
-    // activation rows. us per call, larger tiles against these: Q4_K 4096 x
-    // 14336 at 64 rows 93 / 23, at 256 (1024 tiles) 98 / 72, at 512 107 / 136;
-    // 14336 x 4096 at 64 (896) 35 / 30, at 128 37 / 47; Q6_K 4096 x 4096 at
-    // 256 (1024) 51 / 44, at 512 67 / 81. The 32-block formats, two blocks to
-    // a CU and slower in the larger tiles: Q8_0 4096 x 14336 at 512 (2048
-    // tiles) 244 / 212, 14336 x 4096 at 128 (1792) 78 / 65, at 256 93 / 114.
-    const uint32_t act_tiles = (n + 31) / 32;
-    const uint64_t tiles = uint64_t{(rows + 31) / 32} * act_tiles;
-    // Up to three 256-blocks a row give a wave one block at most: the larger
-    // tiles' one running sum is then as exact (768 columns, error against 64
-    // bits 5.1e-8 in those, 5.2e-8 in these; from four blocks on these have
-    // the smaller one).
-    if (staged && tiles <= (kq ? 1024u : 2048u) && (!kq || cols >= 1024)) {
+    if (kernel == quant_kernel::ks) {
+        const uint32_t act_tiles = (n + 31) / 32;
+        const uint32_t tiles = (rows + 31) / 32 * act_tiles;
         for_qtype(t, [&]<uint32_t T>() {
-            gemm_ks_kernel<T><<<static_cast<uint32_t>(tiles), 256, 0, stream>>>(w, act, bias, out, n, rows, cols,
-                                                                                act_tiles);
+            gemm_ks_kernel<T><<<tiles, 256, 0, stream>>>(w, act, bias, out, n, rows, cols, act_tiles);
         });
         return hipGetLastError();
     }
+    const bool staged = matmul_q_staged(t, w, act, cols);
     const dim3 grid((rows + gq_m - 1) / gq_m, (n + gq_n - 1) / gq_n);
     for_qtype(t, [&]<uint32_t T>() {
         if constexpr (T == qtype_q4_k) {

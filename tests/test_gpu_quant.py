@@ -107,12 +107,14 @@ def test_matmul_q_matches_host_blocks(arena, t, n, rows, cols):
 @pytest.mark.parametrize("n,rows,cols", [(32, 37, 512), (70, 130, 2048), (64, 128, 4096), (33, 300, 256),
                                          (129, 33, 768), (40, 50, 800), (32, 1, 256), (65, 3, 512), (32, 2, 64)])
 def test_matmul_q_gemm_matches_host(arena, t, n, rows, cols):
-    """From 32 activation rows on, the product runs on the int8 matrix cores;
-    the activation bytes stay ggml's bit for bit and every output is within
-    1e-5 of sum |w| |x^| of the exact product of the dequantized operands
-    (each block's integer sum is exact; only float association differs).
-    800 columns (25 blocks, not whole two-block stages) take the 32-block
-    formats' register kernel, the others their LDS kernels."""
+    """From 32 activation rows on, the product runs on the int8 matrix cores in
+    every format; the activation bytes stay ggml's bit for bit and every
+    output is within 1e-5 of sum |w| |x^| of the exact product of the
+    dequantized operands (each block's integer sum is exact; only float
+    association differs). 800 columns (25 blocks, not whole two-block stages)
+    take the 32-block formats' register kernel; of the others these sizes are
+    16-row tiles (32 rows), 32 x 32 tiles, and, below 1024 columns, the K
+    formats' larger tiles."""
     if cols % BLOCK[t][0]:
         pytest.skip("cols not whole blocks")
     rng = np.random.default_rng(7000 + 31 * t + n)
@@ -136,24 +138,28 @@ def test_matmul_q_gemm_matches_host(arena, t, n, rows, cols):
 def test_gemm_at_model_size_matches_the_gemv(arena, t, rows, cols):
     """Llama-3-8B row lengths (ffn_up's 4096 columns, ffn_down's 14336),
     128 activation rows: many workgroups in both dimensions and every stage
-    of a long row (the row counts are cut to keep the host's bound quick). The GEMM (int8 matrix cores,
-    LDS-staged) and the GEMV (v_dot4, one wave per row) are separate kernels
-    over the same exact block integers, so they agree within twice the
-    float-association bound, 2e-5 of sum |w| |x^|; the activation bytes are
-    ggml's bit for bit."""
+    of a long row (the row counts are cut to keep the host's bound quick).
+    128 rows at once (32 x 32 matrix-core tiles), 16 at a time (16-row tiles)
+    and, for the first rows, 2 at a time (the GEMV: v_dot4, one wave per row)
+    are separate kernels over the same exact block integers, so they agree
+    within twice the float-association bound, 2e-5 of sum |w| |x^|; the
+    activation bytes are ggml's bit for bit."""
     rng = np.random.default_rng(9000 + t)
     raw = random_blocks(t, rows, cols, rng)
     n = 128
     x = rng.standard_normal((n, cols)).astype(np.float32)
     gemm, act = matmul_q(arena, raw, t, x, rows, cols)
-    gemv = np.concatenate([matmul_q(arena, raw, t, x[i:i + 16], rows, cols)[0] for i in range(0, n, 16)])
+    tiles16 = np.concatenate([matmul_q(arena, raw, t, x[i:i + 16], rows, cols)[0] for i in range(0, n, 16)])
+    gemv = np.concatenate([matmul_q(arena, raw, t, x[i:i + 2], rows, cols)[0] for i in range(0, 16, 2)])
     want_act = np.concatenate([qh.quantize_act(x[r], t) for r in range(n)])
     assert np.array_equal(act, want_act)
     w_abs = np.abs(qh.dequantize(raw, t).reshape(rows, cols))
     xa = np.abs(np.stack([qh.dequantize_act(a, qh.act_type(t)) for a in want_act.reshape(n, -1)]))
     scale = (xa @ w_abs.T).astype(np.float64)
-    err = np.abs(gemm.astype(np.float64) - gemv.astype(np.float64))
-    assert np.all(err <= 2e-5 * np.maximum(scale, 1.0)), float((err / np.maximum(scale, 1.0)).max())
+    for other in (tiles16, gemv):
+        m = len(other)
+        err = np.abs(gemm[:m].astype(np.float64) - other.astype(np.float64))
+        assert np.all(err <= 2e-5 * np.maximum(scale[:m], 1.0)), float((err / np.maximum(scale[:m], 1.0)).max())
 
 
 @pytest.mark.parametrize("t", [Q4_0, Q5_0, Q8_0, Q4_K, Q6_K])

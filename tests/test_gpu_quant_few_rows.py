@@ -28,11 +28,12 @@ def arena():
 # a tile less one, whole and one over; odd counts start rows off a dword
 # (Q6_K). Columns: one unit (seven waves idle), one per wave, one more, and
 # for the 32-block formats a last unit of two to six blocks, and one of 25
-# blocks (odd: the kernels that copy whole units do not take it).
+# blocks (odd: the kernels that copy whole units do not take it). Long rows of
+# few weight rows, which the GEMV keeps in some formats, and their 16-row tiles.
 CASES = [(2, 17, 512), (3, 1, 256), (3, 15, 2048), (5, 33, 2304), (15, 16, 768), (16, 31, 4096), (17, 16, 256),
          (24, 65, 14336), (31, 5, 2560), (32, 130, 1024), (33, 31, 256), (40, 33, 1280), (64, 65, 1024), (65, 32, 2048),
          (96, 7, 768), (3, 17, 64), (16, 15, 320), (20, 33, 448), (33, 9, 64), (40, 33, 192), (31, 20, 800),
-         (33, 20, 800)]
+         (33, 20, 800), (3, 40, 4352), (3, 1040, 4352), (16, 9, 6400), (16, 600, 6400), (31, 9, 8192)]
 
 
 @pytest.mark.parametrize("t", [Q4_0, Q5_0, Q8_0, Q4_K, Q6_K])
@@ -46,12 +47,33 @@ def test_few_rows(arena, t, n, rows, cols):
     _check(arena, t, n, rows, cols)
 
 
-# The last count of 32 x 32 tiles that gemm_ks_kernel takes, and one row more.
+# Around the counts of 32 x 32 tiles from which gemm_ks_kernel asks for more
+# columns or gives way to the larger tiles (test_quant_plan.cpp pins which
+# kernel each takes).
 @pytest.mark.parametrize("t,rows,cols", [(Q4_K, 16384, 1024), (Q4_K, 16385, 1024), (Q6_K, 16384, 1024),
                                          (Q6_K, 16385, 1024), (Q4_K, 16, 768),
-                                         (Q8_0, 32768, 64), (Q8_0, 32769, 64)])
+                                         (Q8_0, 32768, 64), (Q8_0, 32769, 64), (Q4_K, 12288, 1024),
+                                         (Q4_K, 12289, 1024), (Q4_K, 12289, 3072), (Q8_0, 12288, 64),
+                                         (Q8_0, 12289, 64), (Q8_0, 12289, 192), (Q5_0, 24576, 192),
+                                         (Q5_0, 24576, 256)])
 def test_tile_count_rule(arena, t, rows, cols):
     _check(arena, t, 33, rows, cols)
+
+
+# 32 activation rows of many weight rows: the larger tiles, half of them empty.
+@pytest.mark.parametrize("t,rows,cols", [(Q4_0, 32768, 64), (Q4_K, 32768, 256), (Q6_K, 131072, 256)])
+def test_thirty_two_rows_of_many(arena, t, rows, cols):
+    _check(arena, t, 32, rows, cols)
+
+
+# The larger tiles (gemm_q4k_kernel, gemm_q6k_kernel, gemm_qb32_kernel), past
+# the tile counts that gemm_ks_kernel takes: ten stages of 256 columns, or five
+# of 64, so that both stage buffers are filled and read again; the last tiles
+# hold one activation row and 104 (40) weight rows.
+@pytest.mark.parametrize("t,n,cols", [(Q4_0, 2049, 320), (Q5_0, 2049, 320), (Q8_0, 2049, 320), (Q4_K, 1025, 2560),
+                                      (Q6_K, 1025, 2560)])
+def test_large_tiles(arena, t, n, cols):
+    _check(arena, t, n, 1000, cols)
 
 
 def _check(arena, t, n, rows, cols):

@@ -93,6 +93,12 @@ def test_f32_product_launches_stay_in_range():
     _run("test_matmul_f32_plan")
 
 
+def test_quantized_product_rule():
+    """The quantized product's choice of kernel: what each takes, launches in
+    range, and that the GPU tests' shapes reach the kernels they are for."""
+    _run("test_quant_plan")
+
+
 def test_session_run_allocates_nothing():
     """session::run under a counting operator new, against a C ABI that
     launches nothing (tests/sdk/graph_no_alloc.cpp:199-263 restated)."""
