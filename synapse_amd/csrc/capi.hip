@@ -887,7 +887,7 @@ int syn_hip_self_attention(syn_arena* a, const syn_self_desc* d) {
     f.scale_log2e = d->scale * syn::log2e;
     f.scale = d->scale;
     if (d->in_dtype == SYN_F32 && syn::self_f32_fits(d->n)) {
-        return hip_status(syn::self_f32_mfma_fits(f) ? syn::launch_self_f32_mfma(f, a->stream)
+        return hip_status(syn::self_f32_mfma_takes(f) ? syn::launch_self_f32_mfma(f, a->stream)
                                                      : syn::launch_self_f32(f, a->stream),
                           "self_attention launch");
     }

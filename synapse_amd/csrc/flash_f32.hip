@@ -26,7 +26,8 @@
 // head are dealt to one XCD, whose L2 then holds that head's K and V.
 // Exponentials are expf of the f32 difference to the running max, and
 // their sum is kept in double per lane, as in the row-per-wave kernel
-// (generic.hip) that this replaces for head sizes in whole 16-byte chunks.
+// (generic.hip) that this replaces for head sizes in whole 16-byte chunks,
+// tiny calls apart (self_f32_mfma_takes).
 
 #include "kernels.hpp"
 
@@ -287,14 +288,22 @@ hipError_t launch_hd(const flash_args& a, hipStream_t stream) {
 
 }  // namespace
 
-bool self_f32_mfma_fits(const flash_args& a) {
+bool self_f32_mfma_takes(const flash_args& a) {
     // Rows are read and written 16 bytes at a time (heads of whole 8-dim
     // chunks are aligned by the interface, those of 4, 12, ... dims need not
     // be); a launch takes fewer than 2^32 threads in one dimension.
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    return a.hd % 4 == 0 && aligned(a.q) && aligned(a.k_rows) && aligned(a.v_rows) && aligned(a.out) &&
-           uint64_t{a.n} * a.row * 4 < (uint64_t{1} << 31) &&
-           (uint64_t{a.n} + sf_q - 1) / sf_q * a.n_heads * a.batch < (uint64_t{1} << 24);
+    const bool fits = a.hd % 4 == 0 && aligned(a.q) && aligned(a.k_rows) && aligned(a.v_rows) && aligned(a.out) &&
+                      uint64_t{a.n} * a.row * 4 < (uint64_t{1} << 31) &&
+                      (uint64_t{a.n} + sf_q - 1) / sf_q * a.n_heads * a.batch < (uint64_t{1} << 24);
+    // A few short rows of tiny heads are done by a wave a row before this
+    // kernel's merge is: us in a graph, row per wave against this one, one
+    // head: 4 dims 1 row 2.4 / 3.1, 32 rows 3.3 / 3.4; 8 dims 8 rows 2.8 /
+    // 3.1, 16 rows 3.1 / 3.2, 32 rows 3.6 / 3.3; 12 dims 8 rows 3.1 / 3.1; 16
+    // dims 2 rows 3.2 / 3.2; and while the rows are few: 8 dims, 16 rows, 64
+    // images 3.5 / 3.5, of 12 heads 8.3 / 3.9.
+    const bool tiny = a.hd <= 12 && uint64_t{a.hd} * a.n <= 160 && uint64_t{a.n} * a.n_heads * a.batch <= 1536;
+    return fits && !tiny;
 }
 
 hipError_t launch_self_f32_mfma(const flash_args& a, hipStream_t stream) {

@@ -99,8 +99,8 @@ __global__ __launch_bounds__(64) void generic_kernel(const flash_args a) {
 // order), the probabilities sit in LDS, and lane l then sums output dims
 // l, l + 64, ... over the keys in order. It takes head sizes that are not
 // whole 16-byte chunks (or rows not on one), images of 2^31 bytes and more,
-// and 2^24 16-row tiles and more; the other f32 shapes take the f32 matrix
-// cores (flash_f32.hip), the f16-input and long-image shapes the binary16
+// 2^24 16-row tiles and more, and a few short rows of tiny heads; the other
+// f32 shapes take the f32 matrix cores (flash_f32.hip), the f16-input and long-image shapes the binary16
 // matrix-core kernel.
 __global__ __launch_bounds__(64) void self_f32_kernel(const flash_args a) {
     extern __shared__ float probs[];  // n

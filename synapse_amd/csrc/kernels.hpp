@@ -267,8 +267,8 @@ bool self_f32_fits(uint32_t n);
 hipError_t launch_self_f32(const flash_args& a, hipStream_t stream);
 // The same on the f32 matrix cores (flash_f32.hip): head sizes in whole
 // 16-byte chunks on 16-byte offsets, an image's rows below 2^31 bytes, fewer
-// than 2^24 blocks of 16 query rows.
-bool self_f32_mfma_fits(const flash_args& a);
+// than 2^24 blocks of 16 query rows, and not a few short rows of tiny heads.
+bool self_f32_mfma_takes(const flash_args& a);
 hipError_t launch_self_f32_mfma(const flash_args& a, hipStream_t stream);
 
 // ---- RoPE -------------------------------------------------------------------

@@ -31,13 +31,17 @@ def arena():
 # at and above 1, 4 and 8 tiles, and a wave left without keys (n = 130 with 3
 # tiles a wave). Head sizes: one chunk, each group of the output's tiles (16,
 # 32, 64 dims) whole and cut, both ends of every compiled size, and 6 (the
-# row-per-wave kernel).
+# row-per-wave kernel). The last line: either side of what that kernel keeps of
+# the tiny heads (160 floats of a head, 1536 rows in all).
 @pytest.mark.parametrize("n,batch,heads,hd", [(1, 1, 1, 64), (15, 2, 3, 64), (16, 1, 1, 64), (17, 3, 1, 64),
                                               (63, 1, 2, 64), (65, 2, 2, 64), (128, 1, 3, 64), (130, 1, 3, 64),
                                               (257, 2, 9, 64), (729, 1, 2, 72), (40, 1, 2, 4), (40, 1, 2, 12),
                                               (40, 2, 2, 32), (70, 1, 2, 36), (70, 1, 3, 80), (70, 1, 2, 84),
                                               (70, 1, 2, 96), (70, 1, 2, 100), (70, 1, 2, 128), (70, 1, 2, 132),
-                                              (70, 1, 2, 192), (70, 1, 2, 196), (70, 1, 2, 256), (70, 1, 2, 6)])
+                                              (70, 1, 2, 192), (70, 1, 2, 196), (70, 1, 2, 256), (70, 1, 2, 6),
+                                              (40, 2, 16, 4), (41, 2, 16, 4), (32, 3, 16, 4),
+                                              (33, 3, 16, 4), (20, 1, 3, 8), (21, 1, 3, 8), (13, 4, 2, 12),
+                                              (14, 4, 2, 12), (8, 1, 2, 16)])
 def test_image_f32(arena, n, batch, heads, hd):
     g = wl.rng(1000 * hd + n)
     q, k, v = (wl.normal(g, (batch * n, heads * hd)) for _ in range(3))
