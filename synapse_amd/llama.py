@@ -282,7 +282,8 @@ class DeviceLlama:
 
     # ---- one op each, through the C ABI ---------------------------------------
     # The graph's calls and their descriptors are laid out once, with the
-    # arena; a step sets the token and the position and makes the calls. A
+    # arena; a step sets the token, the position and the KV states of that
+    # moment and makes the calls. A
     # small model's step is bound by these calls on the host: a two-layer F32
     # step of 2048 takes 207-211 us (220 with the descriptors built per call).
     def _call(self, entry, *descs):
@@ -364,7 +365,8 @@ class DeviceLlama:
         handle = self.arena.handle
         tok = (ctypes.c_uint32 * 1)(token)
         check(lib().syn_hip_embed(handle, ctypes.byref(self._embed), tok, 1))
-        for ad in self._attn:
+        for ad, cache in zip(self._attn, self.caches, strict=True):
+            ad.cache = cache  # (a program may give the model another sequence's states)
             ad.pos = pos
         for entry, descs in self._graph:
             status = entry(handle, *descs)
