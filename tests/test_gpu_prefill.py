@@ -91,14 +91,15 @@ def test_prefill_llama3_8b_2048(arena):
     assert_close(got, want, what="C3 all rows")
 
 
-@pytest.mark.parametrize("n,pos", [(2048, 0), (300, 0), (1000, 77)])
+@pytest.mark.parametrize("n,pos", [(2048, 0), (300, 0), (1000, 77), (1300, 0), (1700, 77)])
 def test_prefill_is_deterministic(arena, n, pos):
-    """Two runs of the same attend over the same cache give the same bits:
-    config 3's shape (every 8-wave block merges its later tile's two
-    partials through LDS in a fixed order), an odd tile count (the middle
-    tile, whose block has one tile) and a run after cached rows. The
-    reference pins thread-count invariance bit for bit
-    (tests/sdk/llama_threads.cpp:32-58)."""
+    """Two runs of the same attend over the same cache give the same bits.
+    Pairs of query tiles: config 3's shape (every 8-wave block merges its
+    later tile's two partials through LDS in a fixed order), an odd tile count
+    (1300: the middle tile, whose block has one tile) and a run after cached
+    rows (1700). Keys split inside the block (four partials merged): 300 and
+    1000 queries, without and after cached rows. The reference pins
+    thread-count invariance bit for bit (tests/sdk/llama_threads.cpp:32-58)."""
     n_heads, n_kv, hd = 32, 8, 128
     cfg = wl.Prefill("case", n_heads, n_kv, hd, pos + n, 500000.0)
     q, k, v = wl.prefill_inputs(cfg, seed=n + pos, f16_exact=True)
@@ -177,18 +178,37 @@ def test_prefill_split_keys(arena, n_heads, n_kv, hd, n, pos, dtype):
     assert_close(got, want, what=f"split keys {n_heads}/{n_kv}/{hd} n={n} pos={pos}")
 
 
-def test_prefill_split_keys_ignores_rows_past_the_run(arena):
+# The kernel of pairs of query tiles (more than 512 blocks of 64 queries) over
+# several items of each wave group, at every compiled head size whole or cut:
+# odd and even tile counts, ends on and off 8- and 64-key edges, after cached
+# rows.
+@pytest.mark.parametrize("n_heads,n_kv,hd,n,pos", [
+    (64, 8, 32, 700, 0), (130, 10, 24, 300, 9), (64, 8, 64, 640, 64), (128, 16, 40, 300, 0), (64, 8, 96, 520, 0),
+    (72, 8, 72, 513, 131), (64, 8, 128, 577, 77),
+])
+@pytest.mark.parametrize("dtype", [SYN_F32, SYN_F16])
+def test_prefill_pairs(arena, n_heads, n_kv, hd, n, pos, dtype):
+    assert n_heads * ((n + 63) // 64) > 512 and pos + n >= 128
+    got, want, (dk, dv), ok_k, ok_v = _prefill(arena, n_heads, n_kv, hd, n, pos, seed=n + hd + pos, dtype=dtype)
+    assert np.array_equal(dk, ok_k[:pos + n]) and np.array_equal(dv, ok_v[:pos + n])
+    assert_close(got, want, what=f"pairs {n_heads}/{n_kv}/{hd} n={n} pos={pos}")
+
+
+# Keys split inside the block, and pairs of query tiles.
+@pytest.mark.parametrize("n_heads,n_kv,hd,n,pos", [(4, 2, 128, 61, 90), (64, 8, 64, 530, 91)])
+def test_prefill_ignores_rows_past_the_run(arena, n_heads, n_kv, hd, n, pos):
     """Cache rows at and past pos + n that hold NaN leave the output as is."""
-    n_heads, n_kv, hd, n, pos = 4, 2, 128, 61, 90
     row = n_kv * hd
     g = wl.rng(91)
-    kc, vc = (wl.to_f16_bits(wl.normal(g, (256, row))) for _ in range(2))
+    kc, vc = (wl.to_f16_bits(wl.normal(g, (pos + n + 105, row))) for _ in range(2))
     q = wl.normal(g, (n, n_heads * hd))
     outs = []
     for bits in (0, 0x7E00):
         kc[pos + n:] = vc[pos + n:] = bits
-        c = capi.kv_state(arena, 256, n_kv, hd)
+        mark = arena.top
+        c = capi.kv_state(arena, pos + n + 105, n_kv, hd)
         capi.upload_cache(arena, c, kc, vc)
-        outs.append(attention(arena, c, scratch_for(arena, n_heads, n_kv, hd, 256), q, None, None, pos, n_heads,
-                              hd ** -0.5, append=False))
+        outs.append(attention(arena, c, scratch_for(arena, n_heads, n_kv, hd, pos + n + 105), q, None, None, pos,
+                              n_heads, hd ** -0.5, append=False))
+        arena.top = mark
     assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
