@@ -67,9 +67,12 @@ def test_image_f32_extreme_scores(arena):
     assert np.isnan(got[7]).all()
     rows = np.arange(n) != 7
     # A score of size s carries an error of s * 2^-24 * sqrt(hd) at most,
-    # which its exponential shows as a relative error.
-    top = np.abs((q[rows] @ k.T) * 0.125).max()
-    assert np.abs(got[rows] - want[rows]).max() <= max(BOUND, top * 2.0 ** -24 * 8) * np.abs(want[rows]).max()
+    # which its exponential shows as a relative error: each row and head is
+    # held to its own largest score.
+    heads_of = lambda x: x[rows].reshape(-1, heads, hd)  # noqa: E731
+    top = np.abs(np.einsum("qhd,khd->qhk", heads_of(q).astype(np.float64), k.reshape(n, heads, hd)) * 0.125).max(-1)
+    err = np.abs(heads_of(got) - heads_of(want)).max(-1)
+    assert np.all(err <= np.maximum(BOUND, top * 2.0 ** -24 * 8) * np.abs(heads_of(want)).max(-1))
 
 
 @pytest.mark.parametrize("at", range(4))
