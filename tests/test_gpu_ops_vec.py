@@ -58,12 +58,26 @@ OPS = {"add": capi.SYN_ADD, "mul": capi.SYN_MUL, "silu_mul": capi.SYN_SILU_MUL, 
 @pytest.mark.parametrize("rows,period", [(1, 1), (1, 3), (3, 4), (7, 6), (5, 1024), (1, 14336), (301, 4096)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_elementwise(arena, op, rows, period, shift):
+    _check_elementwise(arena, op, rows, period, shift, shift, shift)
+
+
+# One operand alone off a 16-byte offset (a, b or the result), then more than
+# 4096 blocks of four floats a thread: a second trip of the vector form's grid,
+# with a bias period that is no power of two.
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("rows,period,shifts", [(9, 1028, (1, 0, 0)), (9, 1028, (0, 1, 0)), (9, 1028, (0, 0, 1)),
+                                                (301, 14340, (0, 0, 0))])
+def test_elementwise_offsets_and_second_trip(arena, op, rows, period, shifts):
+    _check_elementwise(arena, op, rows, period, *shifts)
+
+
+def _check_elementwise(arena, op, rows, period, shift_a, shift_b, shift_out):
     g = wl.rng(rows + period)
     a = wl.normal(g, (rows, period), 3.0)
     b = wl.normal(g, (period,) if op == "add_bias" else (rows, period))
     mark = arena.top
-    ao, bo = _put(arena, a, shift), _put(arena, b, shift)
-    oo = _put(arena, np.full(rows * period + 8, 7.0, np.float32), shift)
+    ao, bo = _put(arena, a, shift_a), _put(arena, b, shift_b)
+    oo = _put(arena, np.full(rows * period + 8, 7.0, np.float32), shift_out)
     d = capi.ElementwiseDesc(a_offset=ao, b_offset=bo, out_offset=oo, count=rows * period, op=OPS[op], scalar=1.7,
                              period=period)
     check(lib().syn_hip_elementwise(arena.handle, ctypes.byref(d)))
