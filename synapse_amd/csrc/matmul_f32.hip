@@ -36,8 +36,8 @@ __device__ __forceinline__ float mf_wave_sum(float v) {
 // and this one is held to the reference's logits to 1e-4 by the golden
 // models; 16-byte loads would take another. What the loads need instead is
 // number: 16 weight loads (4 KB) in flight per wave and eight waves per SIMD.
-// One row of 16000 x 2048 21.5 us (6.1 TB/s), 5632 x 2048 8.8, 2048 x 5632
-// 8.9 us; with one load in flight per lane 39.4, 17.7 and 41.0.
+// One row of 16000 x 2048 21.5 us a call (6.1 TB/s), 5632 x 2048 8.0, 2048 x
+// 5632 8.5; with one load in flight per lane 39.4, 12.8 and 29.1.
 // Row resources end at the row, so columns past it add zeros.
 // U loads are in flight per lane: as many as the row has for a lane, at most
 // 16 (a load past the row costs its issue all the same: 20000 x 16 with 3

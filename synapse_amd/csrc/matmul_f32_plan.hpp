@@ -21,9 +21,10 @@ struct matmul_f32_plan {
 // The matrix-core kernel's time for few rows is its stages' latency (6 ns per
 // column), the other's grows with n rows cols (0.15 us per million): they
 // meet at n rows = 40000. us per call, one wave per weight row against
-// tiles: 768 x 3072 weights 12.3 / 19.9 at 32 rows, 22.7 / 22.8 at 64; 3072 x
-// 768 5.9 / 6.7 at 8 and 9.7 / 8.0 at 16; 1152 x 588 7.3 / 7.7 at 32, 12.7 /
-// 8.1 at 64. Fewer than 8 rows would leave three quarters of a tile empty.
+// tiles: 768 x 3072 weights 12.9 / 23.4 at 32 rows, 23.5 / 23.5 at 64; 3072 x
+// 768 5.8 / 7.6 at 8 and 9.4 / 8.0 at 16; 1152 x 588 7.4 / 8.1 at 32, 12.6 /
+// 8.1 at 64; 1024 x 1024 20.9 / 10.6 at 128. Fewer than 8 rows would leave
+// three quarters of a tile empty.
 // The tiled kernel copies whole 16-byte chunks of a row, through 32-bit
 // offsets below 2^31 over a tile's 64 rows.
 constexpr bool matmul_f32_on_matrix_cores(uint32_t n, uint32_t rows, uint32_t cols) {
@@ -37,10 +38,10 @@ constexpr matmul_f32_plan plan_matmul_f32(uint32_t n, uint32_t rows, uint32_t co
     if (matmul_f32_on_matrix_cores(n, rows, cols)) {
         // The largest tile whose count still fills the 256 CUs (the waves
         // then split the columns). us per call for 64 x 64, 32 x 64 and
-        // 32 x 32 tiles (with one running sum): 1024 rows of 3072 x 768 45.4,
-        // 50.4, 60.4 (768 tiles of 64 x 64); 512 rows 31.8, 28.3, 33.7 (384
-        // and 768); 729 rows of 768 x 3072 61.1, 57.9, 53.1 (144, 276, 552);
-        // 257 rows of 768 x 768 18.0, 11.6, 8.1.
+        // 32 x 32 tiles: 1024 rows of 3072 x 768 46.6, 50.6, 64.7 (768 tiles
+        // of 64 x 64); 512 rows 32.5, 26.5, 33.5 (384 and 768); 729 rows of
+        // 768 x 3072 71.7, 62.6, 54.5 (144, 276, 552); 257 rows of 768 x 768
+        // 21.0, 13.0, 8.8.
         const uint32_t bm = tiles(64, 64) >= 512 ? 64 : 32;
         const uint32_t bn = bm == 64 || tiles(32, 64) >= 384 ? 64 : 32;
         if (tiles(bm, bn) < matmul_f32_max_blocks) {

@@ -147,9 +147,10 @@ constexpr bool elementwise_reads_b(uint32_t op) {
 }
 
 // N floats per thread and trip: 4 where everything is 16-byte aligned (and b's
-// period whole chunks), else 1. Latency-bound at decode sizes: SiLU times up
-// over 14336 floats 2.4 us, an add of 4096 2.0, against 3.9 with one kernel
-// for all ops (a switch and a 64-bit remainder in its loop), one float a trip.
+// period whole chunks), else 1. At decode sizes a launch's latency is all there
+// is: SiLU times up over 14336 floats 1.8 us in a graph, an add of 4096 1.8,
+// as with one kernel for all ops (a switch and a 64-bit remainder in its
+// loop), one float a trip; over 2^20 floats 2.5 us, 3.2 so.
 template <uint32_t OP, int N>
 __global__ __launch_bounds__(256) void elementwise_kernel(const float* a, const float* b, float* out, uint64_t count,
                                                           float scalar, uint32_t period) {
@@ -329,9 +330,10 @@ hipError_t launch_rms_norm(const float* in, const float* gamma, float* out, uint
                            hipStream_t stream) {
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     if (size % 4 == 0 && aligned(in) && aligned(gamma) && aligned(out)) {
-        // As few threads as hold the row: one row of 4096 takes 2.2 us with
-        // 256 (2.5 with 1024, 5.5 in the row-loop form), 2048 rows 10.7 (14.3,
-        // 16.9); replayed from a graph.
+        // As few threads as hold the row: one row of 4096 takes 2.1-2.2 us
+        // with 256 (2.5 with 1024, 5.5 in the row-loop form), 2048 rows 9.7-
+        // 10.7 (14.3, 15.2-16.9), one of 16384 3.2 with 1024 (16.6 in the
+        // row-loop form); replayed from a graph.
         // (A launch takes fewer than 2^32 threads.)
         const bool held = size <= 256 * 16 || (size <= 1024 * 16 && n < (1u << 22));
         if (size <= 256 * 4) {

@@ -439,9 +439,13 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void prefill_kernel(const f
 // (max, sum, O) of the later tile's queries meet in LDS at the end, in a
 // fixed order. The tail of the last V^T chunk past kv_end is zeroed by the
 // lane that copied it, right after its copy lands. 2048 queries of 32 heads on
-// 8, hd 128: 56.2 us (59.5-61.4 with two barriers a tile and the row sums
-// taken across the lane halves on every tile), 612 TFLOP/s; what bounds it is
-// the LDS reads (a wave reads a whole tile for 32 queries) beside the softmax.
+// 8, hd 128, back to back: 55.5-58.5 us on different boxes, 587-619 TFLOP/s
+// (on one box 56.2, and 59.5-61.4 with two barriers a tile and the row sums
+// taken across the lane halves on every tile). What bounds it is the chain of
+// a wave's item (scores, max, exponentials and conversions, output products)
+// at two waves per SIMD: the matrix cores are busy 26 % of the time, waves
+// issue in 29 % of their cycles and wait in 36 %, of which 1.6 % on the LDS,
+// whose operand reads take a quarter of its bandwidth.
 template <int HD, bool QF16>
 __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a) {
     constexpr int NS = HD / 16;
@@ -855,8 +859,8 @@ __global__ __launch_bounds__(512, 2) void prefill_pair_kernel(const flash_args a
 // order. One barrier per tile: tile j has landed and tile j - 1 is read, so
 // tile j + 1's copy goes out ahead of tile j's products.
 //
-// 509 queries after 7683 rows (32 heads on 8, hd 128): 112 us, 590 TFLOP/s
-// (263 us as pairs). Copies alone take 81 us (each tile serves 64 queries, so
+// 509 queries after 7683 rows (32 heads on 8, hd 128): 103-106 us a call with
+// its append, 630 TFLOP/s (245 us as pairs). Copies alone take 81 us (each tile serves 64 queries, so
 // the CUs read 1.07 GB through L2) and the products and softmax alone 83:
 // with one block per CU in step they overlap only in part.
 constexpr int ps_bq = 64;  // queries per block
@@ -1217,12 +1221,13 @@ hipError_t launch_hd(const flash_args& a, uint32_t dtype, hipStream_t stream) {
         // Two wave groups' stages fit LDS up to hd 128.
         const dim3 grid(a.n_heads * ((a.n + 2 * pf_bq - 1) / (2 * pf_bq)));
         // Where those blocks leave CUs idle, blocks of 64 queries with the
-        // keys split four ways, up to two of them per CU. us per call, pairs
-        // against split keys (32 heads on 8, hd 128): 509 queries after 7683
-        // rows 263 / 112, after 1000 53 / 25, after none 22.3 / 13.4; 64 after
-        // 7683 127 / 91; 1024 after 7683 (512 blocks) 275 / 211, 1100 after
-        // 7683 (576) 269 / 283. Below 128 keys there is little to split: 64
-        // queries after none 6.9 / 8.2, after 100 9.6 / 9.4.
+        // keys split four ways, up to two of them per CU. us per call with
+        // its append, pairs against split keys (32 heads on 8, hd 128): 509
+        // queries after 7683 rows 245 / 103, after 1000 55 / 29, after none
+        // 26.5 / 17.1; 64 after 7683 119 / 96; 1024 after 7683 (512 blocks)
+        // 255 / 206, 1100 after 7683 (576) 253 / 286. Below 128 keys there is
+        // little to split: 64 queries after none 9.2 / 10.6, after 100 13.1 /
+        // 12.8.
         const uint32_t cus = device_cu_count();
         const dim3 fine(a.n_heads * ((a.n + ps_bq - 1) / ps_bq));
         if (grid.x < cus && fine.x <= 2 * cus && a.kv_len >= 128) {

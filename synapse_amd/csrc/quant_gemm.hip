@@ -923,8 +923,9 @@ __global__ __launch_bounds__(256, 4) void gemm_qb32_kernel(const uint8_t* w, con
 // same whole-line copies and layouts as above, ks_stages deep) and waits for
 // nothing but its copies: no barrier until the four partial sums meet, in a
 // fixed order. The block sums are the same exact integers. 64 rows against
-// Q4_K 4096 x 14336: 23 us a call (93 in the 128 x 64 tiles), Q6_K 34 (121),
-// Q8_0 41 (239).
+// Q4_K 4096 x 14336: 22 us a call (93 in the 128 x 64 tiles), Q6_K 31 (113),
+// Q8_0 40 (220).
+//
 // gemm_q4k_kernel's block for one tile of 32 activation rows: this lane's
 // weight row (its 144 bytes at Wl) against the rows of the stage at S, qs at A
 // (256 bytes a row, 16-byte chunk k of a row at k ^ (row % 16)), the 16 sums
@@ -1277,11 +1278,13 @@ __global__ __launch_bounds__(256) void gemm_ks_kernel(const uint8_t* w, const ui
 //
 // A wave stages 256 columns of its rows in its own LDS, reads all operands
 // into registers, sends the next copies off and only then decodes and
-// multiplies: one stage, no barrier. The eight partial sums meet in a fixed
-// order. 24 rows against Q6_K 4096 x 14336: 22 us a call with the quantizer
-// (48 MB of weights, 2.2 TB/s), 147 us as six passes of the GEMV; bound by
-// the decode (about 300 vector instructions per 16 x 256 weights) and, above
-// 16 rows, one block per CU for its LDS.
+// multiplies: one stage, no barrier. (In the 32-block formats the next copies
+// go out behind the unit's products, and each unit waits them out: about 2 us
+// per 2048 columns.) The eight partial sums meet in a fixed order. 24 rows
+// against Q6_K 4096 x 14336: 18.8 us a call with the quantizer (48 MB of
+// weights, 2.6 TB/s), 147 us as six passes of the GEMV; bound by the decode
+// (about 300 vector instructions per 16 x 256 weights) and, above 16 rows,
+// one block per CU for its LDS.
 
 template <uint32_t T>
 struct r16_layout {
